@@ -39,7 +39,8 @@
 //     XCDs per stream the heads of each tile pair are dealt over that set in turn,
 //     which keeps the XCDs' shares of the work equal. Given a work queue, the grid
 //     is persistent: one workgroup per CU takes its XCD's items in that order from
-//     a counter, then the light last third of the tile pairs from a shared one.
+//     a counter, then the light last third of the tile pairs from a shared one, then
+//     what is left of the other XCDs' items.
 #include <type_traits>
 
 #include "common.h"
@@ -83,12 +84,15 @@ struct AttnArgs {
   int xcds_per_stream;   // XCDs sharing one (batch, kv group) stream; 1: pair p on XCD p % 8
   float scale_log2;
   // Persistent grid (a caller queue): one workgroup per CU takes items until none
-  // are left. Tile pairs [0, static_tp) are dealt to XCDs as in the static grid and
-  // taken in order through XCD x's counter queue[1 + x]; the rest (the lightest) go
-  // through queue[0] in heaviest-first order to whichever XCD asks first.
+  // are left (draw_item). Tile pairs [0, static_tp) are dealt to XCDs as in the static
+  // grid and taken in order through XCD x's counter queue[1 + x]; the rest (the
+  // lightest) go through the tail counters in heaviest-first order.
   int* queue;        // SPX_WORK_QUEUE_INTS zeroed int32 (null: one workgroup per item)
   int static_tp;     // tile pairs on the per-XCD deal (all of them without a queue)
-  int dyn_items;     // (tile pair, stream, head) items of the shared tail
+  int steal;         // workgroups also take items of other XCDs' static shares
+  int share_items;   // xcds_per_stream > 1: items of each XCD's static share
+  int dyn_items;     // items behind each tail counter: (tile pair, head) of one stream
+                     // (xcds_per_stream > 1), else (tile pair, stream, head)
 };
 
 __device__ __forceinline__ int swz(int row, int chunk) {
@@ -681,6 +685,118 @@ __device__ __forceinline__ void copy_q(const AttnArgs& a, int b, int h, int t0, 
 template <bool EXACT, bool TAIL, bool OUT_F32>
 __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg);
 
+// Items of XCD `xcd`'s share of the static deal.
+__device__ __forceinline__ int static_share(const AttnArgs& a, int xcd) {
+  return a.xcds_per_stream > 1 ? a.share_items
+                               : ((a.static_tp * a.batch * a.kv_heads - xcd + 7) >> 3) * a.group;
+}
+
+// The workgroup's next item, drawn by its first wave (all 64 lanes call this);
+// pair = -1 when none is left. The masks (kept in LDS, so that no register holds them
+// across items) have bit i set once this workgroup found counter i used up (spent), and
+// once it drew from it in vain (drawn).
+//
+// Order: own XCD's static share; the shared light tail, or with 8 / bg XCDs per stream
+// that of its own stream (whose K / V tiles its L2 holds); then, from one look at all
+// counters, the static share of another XCD with the most items left; then the other
+// tails. (Shares before the tail cost balanced layers a look at the counters per stolen
+// item: four 2113-token sequences 225 -> 231 us.) Routed lists differ in length from head
+// to head and group to group by far more than XCD speeds do: without the steals a layer
+// ended with the XCDs of its densest kv group alone (heads selecting 10 to 100 % of the
+// blocks: layer of 131072 tokens 78.0 -> 42.7 ms, of 32640 tokens 2.49 -> 1.84 ms).
+//
+// A draw past the end of another XCD's share is given back, and what a workgroup never
+// drew from its own share and the tails is drawn once when it ends, so the final
+// counters do not depend on who took what: a share's counter ends at its items plus its
+// own XCD's workgroups, a tail's at its items plus the grid.
+__device__ __forceinline__ void draw_item(const AttnArgs& a, int xcd, uint32_t& spent,
+                                          uint32_t& drawn, int& pair, int& hg) {
+  const int lane = thread_x() & 63;
+  const int bg = a.batch * a.kv_heads;
+  const bool per_stream = a.xcds_per_stream > 1;
+  const int own = 1 + xcd, own_tail = per_stream ? kStreamCounter0 + xcd % bg : 0;
+  const uint32_t tails = per_stream ? ((1u << bg) - 1u) << kStreamCounter0 : 1u;
+  pair = -1;
+  if (!((spent >> own) & 1u)) {
+    int d = 0;
+    if (lane == 0) d = atomicAdd(a.queue + own, 1);
+    d = __builtin_amdgcn_readfirstlane(d);
+    if (d < static_share(a, xcd)) {
+      static_item(a, xcd, d, pair, hg);
+      return;
+    }
+    spent |= 1u << own;
+    drawn |= 1u << own;
+  }
+  // items behind this lane's counter (0: not a counter of this launch)
+  int items = 0;
+  if (lane >= 1 && lane <= 8) items = static_share(a, lane - 1);
+  else if (lane < SPX_WORK_QUEUE_INTS && ((tails >> lane) & 1u)) items = a.dyn_items;
+  uint32_t open = 0;     // counters with items left at the last look
+  int left = 0;
+  for (;;) {
+    int c = -1;   // the counter to draw from
+    if (!((spent >> own_tail) & 1u)) {
+      c = own_tail;
+    } else {
+      if (a.steal) {
+        left = 0;
+        if (items > 0 && !((spent >> lane) & 1u))
+          left = items - __hip_atomic_load(a.queue + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        open = (uint32_t)__ballot(left > 0);
+        spent |= ~open;
+      } else {
+        open = tails & ~spent;
+      }
+      if ((open >> 1) & 0xffu) {
+        int best = (lane >= 1 && lane <= 8 && left > 0) ? left * 16 + lane : 0;
+#pragma unroll
+        for (int o = 8; o >= 1; o >>= 1) best = max(best, __shfl_xor(best, o));
+        c = __builtin_amdgcn_readfirstlane(best) & 15;
+      } else if (open & tails) {
+        // the tails in turn from the own one on
+        const uint32_t from_own = (open & tails) >> own_tail;
+        c = from_own ? own_tail + __builtin_ctz(from_own) : __builtin_ctz(open & tails);
+      } else {
+        if (lane < SPX_WORK_QUEUE_INTS && (((((1u << own) | tails) & ~drawn) >> lane) & 1u))
+          atomicAdd(a.queue + lane, 1);
+        return;
+      }
+    }
+    int d = 0;
+    if (lane == 0) d = atomicAdd(a.queue + c, 1);
+    d = __builtin_amdgcn_readfirstlane(d);
+    const int n = __builtin_amdgcn_readlane(items, c);
+    if (d < n) {
+      if (c >= 1 && c <= 8) {
+        static_item(a, c - 1, d, pair, hg);
+      } else if (per_stream) {
+        const int tpk = d / a.group;
+        hg = d - tpk * a.group;
+        pair = (a.static_tp + tpk) * bg + (c - kStreamCounter0);
+      } else {
+        tail_item(a, d, pair, hg);
+      }
+      return;
+    }
+    if (c >= 1 && c <= 8 && lane == 0) atomicSub(a.queue + c, 1);
+    spent |= 1u << c;
+    drawn |= 1u << c;
+  }
+}
+
+// The kernel arguments, read afresh through an opaque pointer.
+__device__ __forceinline__ AttnArgs fresh_args(const AttnArgs& args) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __attribute__((address_space(4))) AttnArgs* ap =
+      (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ap));
+  return *ap;
+#else
+  return args;
+#endif
+}
+
 // Workgroup i runs on XCD i % 8. Without a queue every workgroup runs the one item
 // the static deal gives it. With one, the grid is persistent: launching a workgroup
 // costs a few microseconds, and each XCD starts its workgroups in blockIdx order, a
@@ -691,75 +807,37 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg);
 template <bool EXACT, bool TAIL, bool OUT_F32>
 __global__ __launch_bounds__(kAttnThreads, 1) void attn_kernel(AttnArgs args) {
   const int xcd = blockIdx.x & 7;
-  __shared__ int next_item;
-  // thread 0's draw state, kept in LDS so that no register holds it across items:
-  // this XCD's share used up; streams of the tail tried
-  __shared__ int share_done, steal;
-  if (threadIdx.x == 0) share_done = steal = 0;
+  __shared__ int next_pair, next_hg;
+  __shared__ uint32_t spent_mask, drawn_mask;   // first wave's, read back by itself
+  if (threadIdx.x == 0) spent_mask = drawn_mask = 0u;
   for (int round = 0;; ++round) {
-    // The arguments are read afresh for every item through an opaque pointer, so
+    // The arguments are read afresh for every item, and again after its draw, so
     // nothing derived from them is held in registers across items.
-#if defined(__HIP_DEVICE_COMPILE__)
-    const __attribute__((address_space(4))) AttnArgs* ap =
-        (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(ap));
-    const AttnArgs a = *ap;
-#else
-    const AttnArgs a = args;
-#endif
     int pair, hg;
-    if (a.queue == nullptr) {
-      if (round > 0) break;
-      static_item(a, xcd, blockIdx.x >> 3, pair, hg);
-    } else {
-      const int bg = a.batch * a.kv_heads;
-      const int n_static = a.xcds_per_stream > 1
-          ? a.static_tp * a.group / a.xcds_per_stream
-          : max(0, (a.static_tp * bg - xcd + 7) / 8) * a.group;
-      // With 8 / bg XCDs per stream, the tail is drawn per stream: a workgroup takes
-      // its own stream's light items first (their K / V tiles are in its L2), then
-      // those of the other streams once its own are gone.
-      const bool per_stream = a.xcds_per_stream > 1;
-      const int stream_items = (a.blocks + 1) / 2 - a.static_tp;   // tile pairs ..
-      const int per_stream_items = stream_items * a.group;        // .. x heads
-      if (threadIdx.x == 0) {
-        int k = -1;
-        if (!share_done) {
-          const int d = atomicAdd(a.queue + 1 + xcd, 1);
-          if (d < n_static) k = d;
-          else share_done = 1;
+    if (args.queue != nullptr) {
+      if (thread_x() < 64) {
+        const AttnArgs a = fresh_args(args);
+        uint32_t spent = __builtin_amdgcn_readfirstlane(spent_mask);
+        uint32_t drawn = __builtin_amdgcn_readfirstlane(drawn_mask);
+        int p = -1, x = 0;
+        draw_item(a, xcd, spent, drawn, p, x);
+        if (thread_x() == 0) {
+          next_pair = p;   // -1: no items left
+          next_hg = x;
+          spent_mask = spent;
+          drawn_mask = drawn;
         }
-        if (k < 0 && per_stream) {
-          for (; steal < bg; ++steal) {
-            const int st = (xcd + steal) % bg;
-            const int d = atomicAdd(a.queue + kStreamCounter0 + st, 1);
-            if (d < per_stream_items) {
-              k = n_static + st * per_stream_items + d;
-              break;
-            }
-          }
-        } else if (k < 0) {
-          const int d = atomicAdd(a.queue, 1);
-          if (d < a.dyn_items) k = n_static + d;
-        }
-        next_item = k;   // -1: no items left
       }
       block_sync();
-      const int k = next_item;
+      pair = __builtin_amdgcn_readfirstlane(next_pair);
+      hg = __builtin_amdgcn_readfirstlane(next_hg);
       block_sync();  // read by every wave before thread 0 takes the next one
-      if (k < 0) break;
-      if (k < n_static) {
-        static_item(a, xcd, k, pair, hg);
-      } else if (per_stream) {
-        const int st = (k - n_static) / per_stream_items;
-        const int d = (k - n_static) - st * per_stream_items;
-        const int tpk = a.static_tp + d / a.group;
-        hg = d - (tpk - a.static_tp) * a.group;
-        pair = tpk * bg + st;
-      } else {
-        tail_item(a, k - n_static, pair, hg);
-      }
+      if (pair < 0) break;
+    } else if (round > 0) {
+      break;
     }
+    const AttnArgs a = fresh_args(args);
+    if (a.queue == nullptr) static_item(a, xcd, blockIdx.x >> 3, pair, hg);
     attn_item<EXACT, TAIL, OUT_F32>(a, pair, hg);
   }
 }
@@ -1163,6 +1241,8 @@ struct AttnRequest {
 // Persistent grid: the last third of the tile pairs (the lightest: their lists are
 // the shortest) form the shared tail.
 constexpr int kStaticThirds = 2;
+// Steals with more streams than XCDs: from this many static items per workgroup on.
+constexpr int kStealItems = 4;
 
 // Workgroups per XCD of the persistent grid: one per CU (the kernel's LDS and
 // registers admit one workgroup per CU).
@@ -1277,7 +1357,16 @@ int launch_attention(const AttnRequest& req, const void* q, const int64_t* q_str
     while (tp0 > 0 && a.xcds_per_stream > 1 && (tp0 * a.group) % a.xcds_per_stream) --tp0;
     a.queue = req.work_queue;
     a.static_tp = tp0;
-    a.dyn_items = (np - tp0) * streams * a.group;
+    // Steals pay as soon as an XCD serves one stream (28/4 heads, routed lists: 6000
+    // tokens 211 -> 204 us, 16000 799 -> 689 us; every block listed: no change). With
+    // more streams than XCDs each XCD already mixes several, and the look at the counters
+    // that ends each workgroup costs more than it finds until a share is several items
+    // per workgroup (32/8 heads: 4 x 2113 tokens, 3 items, 225 -> 227 us; 4 x 4500
+    // tokens, 6 items, 546 -> 534 us; 2 x 9000, 6 items, 831 -> 730 us).
+    a.steal = a.xcds_per_stream > 1 ||
+              tp0 * streams / 8 * a.group > kStealItems * persistent_per_xcd();
+    a.share_items = tp0 * a.group / a.xcds_per_stream;
+    a.dyn_items = (np - tp0) * a.group * (a.xcds_per_stream > 1 ? 1 : streams);
     grid = 8 * std::min(persistent_per_xcd(), per_xcd);
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
