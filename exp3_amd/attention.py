@@ -18,16 +18,21 @@ runs entirely in gfx950 HIP kernels:
               spx_sparse_attention_rescue  same, with the rescue tail fused in
 
 so the reference's separate "merge" stage (and, for the mean methods, its "mean"
-stage) takes no time here and is reported as 0 ms. Dense prefill and every decode step use
+stage) takes no time here and is reported as 0 ms. Dense prefill uses
 ``F.scaled_dot_product_attention`` exactly as the reference does
 (attention.py:179-189); ``dense_impl="hip"`` routes dense prefill through the
-HIP kernel with implicit all-causal block lists instead.
+HIP kernel with implicit all-causal block lists instead. A decode step (one query
+row, bf16, head dim 128 or 256) runs in spx_decode_attention; every other
+non-prefill call goes to SDPA as in the reference.
 """
 
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 import torch.nn.functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib, kernels
 from .kernels import BlockDescriptors
@@ -61,6 +66,43 @@ STAGE_NAMES = ("descriptor", "selector", "indices", "exact", "mean", "merge", "a
 
 def _blocks(sequence: int, block_size: int) -> int:
     return (sequence + block_size - 1) // block_size
+
+
+def _decode_kernel_takes(query, key, value, scaling) -> bool:
+    """Whether a non-prefill call is a decode step of spx_decode_attention: one query
+    row per head of plain bf16 GPU tensors in a layout it reads in place, and nothing
+    around the call that SDPA honours and a raw kernel cannot (autograd in either
+    mode, autocast, tracing and function transforms, a backend pin without flash).
+    SDPA runs one workgroup per head (28/4 heads: 1156 us behind 32K tokens, 150 behind
+    4K); at 130 tokens both are bound by the host's launches, so the length does not
+    decide."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._functorch.maybe_current_level() is not None
+            or torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0
+            or any(type(mode) is not DeviceContext       # a default device: factories only
+                   for mode in _get_current_function_mode_stack())
+            or torch.is_autocast_enabled("cuda") or not torch.backends.cuda.flash_sdp_enabled()):
+        return False
+    if not isinstance(scaling, (int, float)):
+        return False
+    device = torch._C._cuda_getDevice() if query.is_cuda else -2
+    for x in (query, key, value):
+        if type(x) is not torch.Tensor or x.get_device() != device \
+                or x.dtype is not torch.bfloat16 or x.dim() != 4:
+            return False
+        batch, heads, rows, dim = x.stride()
+        if dim != 1 or (batch | heads | rows) & 7 or x.data_ptr() & 15:
+            return False
+    batch, q_heads, rows, head_dim = query.shape
+    shape = key.shape
+    if rows != 1 or head_dim not in (128, 256) or shape != value.shape or 0 in shape \
+            or shape[0] != batch or shape[3] != head_dim or q_heads % shape[1] \
+            or batch * q_heads > 65535:
+        return False
+    if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad
+                                    or value.requires_grad):
+        return False
+    return True
 
 
 class AttentionBackend:
@@ -252,6 +294,20 @@ class AttentionBackend:
         _, _, tiles = self._pool(k, v, False, False, True)
         return self._attention(q, k, tiles, None, None, scale, None, want_lse=False)
 
+    @staticmethod
+    def _decode(query, key, value, scale):
+        """One query row per head against the whole cache -> [B, 1, Hq, D]."""
+        batch, q_heads, _, head_dim = query.shape
+        _, kv_heads, sequence, _ = key.shape
+        nbytes = _lib.load().spx_decode_workspace_bytes(batch, sequence, q_heads, kv_heads, head_dim)
+        workspace = query.new_empty(nbytes, dtype=torch.uint8) if nbytes else None
+        output = query.new_empty(batch, 1, q_heads, head_dim)
+        _lib.call("spx_decode_attention", _lib.ptr(query), _lib.strides(query), _lib.ptr(key),
+                  _lib.strides(key), _lib.ptr(value), _lib.strides(value), batch, sequence,
+                  q_heads, kv_heads, head_dim, scale, _lib.ptr(workspace), _lib.ptr(output),
+                  _lib.stream(query.device))
+        return output
+
     def forward(
         self,
         module,
@@ -278,7 +334,9 @@ class AttentionBackend:
             overall_start.record()
 
         is_prefill = query.shape[2] == key.shape[2]
-        if (self.method == "dense" and self.dense_impl == "sdpa") or not is_prefill:
+        if not is_prefill and _decode_kernel_takes(query, key, value, scaling):
+            output = self._decode(query, key, value, float(scaling))
+        elif (self.method == "dense" and self.dense_impl == "sdpa") or not is_prefill:
             output = F.scaled_dot_product_attention(
                 query, key, value, attn_mask=None, dropout_p=0.0, is_causal=is_prefill,
                 scale=scaling, enable_gqa=True,

@@ -38,7 +38,7 @@ extern "C" {
 #define SPX_EUNSUPPORTED (-2) /* valid in the reference, not built here       */
 #define SPX_ELAUNCH (-3)      /* HIP launch / runtime failure                 */
 
-#define SPX_ABI_VERSION 8
+#define SPX_ABI_VERSION 9
 
 /* int32 counters a work_queue argument of the attention entry points points to. */
 #define SPX_WORK_QUEUE_INTS 16
@@ -299,6 +299,21 @@ int spx_sparse_attention_rescue(const void* q, const int64_t* q_strides, const v
                                 const int64_t* out_strides, float* lse,
                                 const int64_t* lse_strides, int32_t* work_queue,
                                 void* stream);
+
+/* --------------------------------------------------------------- decode */
+
+/* One decode step: softmax(scale q K^T) V over the whole KV cache for one query row
+ * per head. q: bf16 [B, Hq, 1, D], k / v: bf16 [B, Hkv, S, D] (strides in that order:
+ * batch, head, sequence, dim), 16-byte aligned bases, batch / head / sequence strides
+ * multiples of 8 elements; out: contiguous bf16 [B, 1, Hq, D], 16-byte aligned.
+ * B * Hq <= 65535. workspace: device memory of spx_decode_workspace_bytes(...) bytes
+ * (-1: unsupported shape; 0: none needed, may be NULL), 16-byte aligned, contents
+ * undefined before and after. Replaces the non-prefill branch of attention.py:179-189. */
+int64_t spx_decode_workspace_bytes(int batch, int seq, int q_heads, int kv_heads, int head_dim);
+int spx_decode_attention(const void* q, const int64_t* q_strides, const void* k,
+                         const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                         int batch, int seq, int q_heads, int kv_heads, int head_dim, float scale,
+                         void* workspace, void* out, void* stream);
 
 /* ----------------------------------------------------------- accounting */
 

@@ -1,0 +1,52 @@
+"""Decode steps on the host: the calls the kernel does not take still go to SDPA, and
+the C entry points refuse what they cannot run before any launch."""
+
+import ctypes
+
+import pytest
+import torch
+
+from exp3_amd import _lib, attention
+
+
+class _Layer:
+    layer_idx = 0
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
+@pytest.mark.parametrize("rows", (1, 3))
+def test_cpu_step_goes_to_sdpa(dtype, rows):
+    gen = torch.Generator().manual_seed(1)
+    q = torch.randn(2, 4, rows, 128, generator=gen).to(dtype)
+    k = torch.randn(2, 2, 40, 128, generator=gen).to(dtype)
+    v = torch.randn(2, 2, 40, 128, generator=gen).to(dtype)
+    assert not attention._decode_kernel_takes(q, k, v, 0.1)
+    backend = attention.AttentionBackend(register=False)
+    backend.configure("fp_v1")
+    out, _ = backend.forward(_Layer(), q, k, v, attention_mask=None, scaling=0.1)
+    wide = [x.double().repeat_interleave(2, 1) for x in (k, v)]
+    want = torch.softmax(q.double() @ wide[0].transpose(2, 3) * 0.1, -1) @ wide[1]
+    torch.testing.assert_close(out.double(), want.transpose(1, 2), rtol=1e-2, atol=1e-2)
+
+
+def test_entry_point_validation():
+    lib = _lib.load()
+    s4 = (ctypes.c_int64 * 4)(4096, 512, 128, 1)
+    odd = (ctypes.c_int64 * 4)(4096, 512, 132, 1)
+    fake, off = 1 << 20, (1 << 20) + 8
+
+    def call(q=fake, k=fake, ks=s4, shape=(1, 600, 28, 4, 128), workspace=fake):
+        return lib.spx_decode_attention(q, s4, k, ks, fake, s4, *shape, 0.1, workspace, fake, None)
+
+    assert call(shape=(1, 600, 28, 4, 64)) == _lib.SPX_EUNSUPPORTED
+    assert call(shape=(1, 600, 28, 3, 128)) == _lib.SPX_EINVAL
+    assert call(shape=(1, 0, 28, 4, 128)) == _lib.SPX_EINVAL
+    assert call(shape=(4096, 600, 28, 4, 128)) == _lib.SPX_EINVAL      # 114688 rows
+    assert call(q=None) == call(k=off) == call(ks=odd) == _lib.SPX_EINVAL
+    assert call(workspace=None) == _lib.SPX_EINVAL                     # three ranges
+    # ranges x rows x (dim + 2) floats; none up to two steps (512 keys, 256 at dim 256)
+    size = lib.spx_decode_workspace_bytes
+    assert size(1, 512, 28, 4, 128) == 0 and size(1, 513, 28, 4, 128) == 3 * 28 * 130 * 4
+    assert size(1, 256, 16, 4, 256) == 0 and size(2, 257, 16, 4, 256) == 3 * 32 * 258 * 4
+    assert size(1, 131072, 28, 4, 128) == 256 * 28 * 130 * 4
+    assert size(1, 512, 28, 4, 64) == size(0, 512, 28, 4, 128) == -1
