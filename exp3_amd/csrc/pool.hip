@@ -11,12 +11,18 @@
 //     position c ^ (r & 15). The attention kernel copies a tile into LDS verbatim
 //     (direct global->LDS loads) and reads MFMA operands bank-conflict free.
 //
-// Bandwidth-bound: each workgroup streams a 128 x D bf16 K tile and V tile with
-// 16-byte loads (each row is 2 D contiguous bytes), reduces columns in registers,
-// across lanes and across the four waves through LDS. The V transpose stages one
-// 64-key half of the rows in LDS at a time (the value slot permutation keeps slots
-// 0-63 on keys 0-63), 25 KB of LDS per workgroup at D = 128: four workgroups per
-// CU, so a 32K-token layer's 1020 workgroups run in one round.
+// Bandwidth-bound at 32K tokens (134 MB with the tiles), latency-bound below (nine
+// blocks at 1089 tokens: 36 workgroups). Half of a workgroup's waves take the K rows,
+// the other half the V rows. Thread = 8 dims x the 16 rows of one value-slot chunk: all
+// 16 of its 16-byte loads are in flight at once, and V is transposed in its registers
+// (the 16 rows are exactly two 8-slot chunks of each of its dims); the finished value
+// tile passes through LDS in 16-byte pieces so that it leaves in whole cache lines
+// (stored from the registers, 16 bytes of each of 64 line parts per instruction: 34.5 us
+// at 32K). Against the form before it, which ran K and V in the same threads and
+// transposed V through LDS in 2-byte reads, same bits (tiles and descriptors, 4 KV
+// heads): 1089 tokens 8.5 -> 5.0 us, 4096 9.1 -> 5.7, 32640 24.2 -> 21.8 (6.2 TB/s),
+// 131072 111 -> 108; 4 x 2113, 8 heads, 16.5 -> 13.7; D = 256, 12001 tokens, 22.3 -> 18.7;
+// descriptors alone at 32640 tokens 14.8 -> 12.6.
 //
 // Head dim 256 (Qwen3.5 full-attention layers): the same pass; key tiles keep the
 // [128 keys][256 dims] layout (chunk c of row r at c ^ (r & 15), c < 32), value tiles
@@ -42,8 +48,6 @@ struct PoolArgs {
   uint16_t* value_tiles;  // [B, Hkv, NB, D, 128]
 };
 
-constexpr int kPoolThreads = 256;
-
 __device__ __forceinline__ void accumulate8(const u32x4& raw, float* sum, float* sq) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -56,150 +60,160 @@ __device__ __forceinline__ void accumulate8(const u32x4& raw, float* sum, float*
   }
 }
 
-// Sum a per-lane array of 8 floats over the row groups of a wave: lanes that differ
-// in bits 4 and 5 (D = 128: 16 chunks per row) or in bit 5 (D = 256: 32 chunks).
+// Value-tile words: the low / high halves of a (low word) and b.
+__device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x05040100u);
+}
+__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+
+constexpr int kPoolRows = 16;                        // rows per thread
+
+// Columns sums of one operand over the block: part[0] / part[1] hold four row-quarter
+// sums of x and x^2 per dim. The order of additions: within a quarter (32 rows) the two
+// 16-row groups' sums, each a chain over its rows (two 8-row chains added at D = 128).
 template <int D>
-__device__ __forceinline__ void reduce_row_groups(float* x) {
+__device__ __forceinline__ void column_sums(const u32x4 (&raw)[kPoolRows], int c, int rg, int lane,
+                                            float (&part)[2][4][D]) {
+  constexpr int kChains = D == 128 ? 2 : 1;
+  float sum[8], sq[8];
+#pragma unroll
+  for (int h = 0; h < kChains; ++h) {
+    float s[8] = {}, q[8] = {};
+#pragma unroll
+    for (int i = 0; i < kPoolRows / kChains; ++i) accumulate8(raw[h * (kPoolRows / kChains) + i], s, q);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      sum[e] = h ? sum[e] + s[e] : s[e];
+      sq[e] = h ? sq[e] + q[e] : q[e];
+    }
+  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    if (D == 128) x[e] += __shfl_xor(x[e], 16);
-    x[e] += __shfl_xor(x[e], 32);
+    sum[e] += __shfl_xor(sum[e], 8);
+    sq[e] += __shfl_xor(sq[e], 8);
+  }
+  if (!(rg & 1)) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      *reinterpret_cast<f32x4*>(&part[0][rg >> 1][c * 8 + e]) =
+          f32x4{sum[e], sum[e + 1], sum[e + 2], sum[e + 3]};
+      *reinterpret_cast<f32x4*>(&part[1][rg >> 1][c * 8 + e]) =
+          f32x4{sq[e], sq[e + 1], sq[e + 2], sq[e + 3]};
+    }
   }
 }
 
+// D threads per operand: K first (if DO_K or DO_TILES), then V (if DO_V or DO_TILES).
 template <int D, bool DO_K, bool DO_V, bool DO_TILES>
-__global__ __launch_bounds__(kPoolThreads) void pool_kernel(PoolArgs a) {
-  constexpr int kChunks = D / 8;                    // 16-byte chunks per row
-  constexpr int kRowsPer = kBlock * kChunks / kPoolThreads;  // rows per row group
-  constexpr int kVPitch = D + 2;                    // LDS row pitch (bf16) of staged V
+__global__ __launch_bounds__(2 * D, 512 / D) void pool_kernel(PoolArgs a) {
+  constexpr bool kReadK = DO_K || DO_TILES, kReadV = DO_V || DO_TILES;
   const int j = blockIdx.x;
   const int b = blockIdx.y / a.kv_heads;
   const int g = blockIdx.y % a.kv_heads;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int c = tid & (kChunks - 1);  // 8-dim chunk
-  const int rg = tid / kChunks;       // row group: rows rg * kRowsPer + i
+  const int lane = tid & 63;
+  // which operand this wave takes, and its thread index there
+  const bool is_v = kReadV && (!kReadK || __builtin_amdgcn_readfirstlane(tid) >= D);
+  const int tx = kReadK && is_v ? tid - D : tid;
+  const int c = (tx >> 6) * 8 + (lane & 7);   // 8-dim chunk
+  const int rg = lane >> 3;                   // row group: rows rg * 16 + i
   const int n = min(kBlock, a.seq - j * kBlock);
 
-  __shared__ float part[4][4][D];                          // [quantity][wave][dim]
-  __shared__ __align__(16) uint16_t vrows[kBlock / 2 * kVPitch];  // staged V rows, one half at a time
-  __shared__ float sig_part[D / 64];
+  __shared__ __align__(16) float part_s[2][2][4][D];   // [K, V][x, x^2][quarter][dim]
+  __shared__ __align__(16) uint16_t vtile[DO_TILES ? kBlock * D : 8];   // the value tile
+  // (40 KB at D = 128: four workgroups per CU; the V wave's sigma goes where its own
+  // first thread's column sum was)
+  auto& part = part_s[is_v && kReadK];
 
-  float sk[8] = {}, qk[8] = {}, sv[8] = {}, qv[8] = {};
-  const uint16_t* kbase = a.k + b * a.ks_b + g * a.ks_h + (int64_t)c * 8;
-  const uint16_t* vbase = a.v + b * a.vs_b + g * a.vs_h + (int64_t)c * 8;
   const int64_t tile_off = ((((int64_t)b * a.kv_heads + g) * a.blocks + j) * kBlock) * D;
-  u32x4 vraw[kRowsPer];   // this thread's V rows (all in one half of the block)
-
+  u32x4 raw[kPoolRows];
+  if (kReadK || kReadV) {
+    const uint16_t* base = is_v ? a.v + b * a.vs_b + g * a.vs_h : a.k + b * a.ks_b + g * a.ks_h;
+    const int64_t stride = is_v ? a.vs_s : a.ks_s;
+    base += (int64_t)j * kBlock * stride + c * 8;
 #pragma unroll
-  for (int i = 0; i < kRowsPer; ++i) {
-    const int row = rg * kRowsPer + i;
-    const bool valid = row < n;
-    const int64_t token = (int64_t)j * kBlock + row;
-    if (DO_K || DO_TILES) {
-      u32x4 raw = {0u, 0u, 0u, 0u};
-      if (valid) raw = *reinterpret_cast<const u32x4*>(kbase + token * a.ks_s);
-      if (DO_K && valid) accumulate8(raw, sk, qk);
-      if (DO_TILES)
-        *reinterpret_cast<u32x4*>(a.key_tiles + tile_off + row * D + ((c ^ (row & 15)) << 3)) = raw;
-    }
-    if (DO_V || DO_TILES) {
-      u32x4 raw = {0u, 0u, 0u, 0u};
-      if (valid) raw = *reinterpret_cast<const u32x4*>(vbase + token * a.vs_s);
-      if (DO_V && valid) accumulate8(raw, sv, qv);
-      if (DO_TILES) vraw[i] = raw;
-    }
-  }
-
-  if (DO_K) { reduce_row_groups<D>(sk); reduce_row_groups<D>(qk); }
-  if (DO_V) { reduce_row_groups<D>(sv); reduce_row_groups<D>(qv); }
-  if (lane < kChunks) {
+    for (int i = 0; i < kPoolRows; ++i)   // rows past the end: the last row, zeroed below
+      raw[i] = *reinterpret_cast<const u32x4*>(base + min(rg * kPoolRows + i, n - 1) * stride);
+    if (n < kBlock) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int d = c * 8 + e;
-      if (DO_K) { part[0][wave][d] = sk[e]; part[1][wave][d] = qk[e]; }
-      if (DO_V) { part[2][wave][d] = sv[e]; part[3][wave][d] = qv[e]; }
+      for (int i = 0; i < kPoolRows; ++i)
+        if (rg * kPoolRows + i >= n) raw[i] = u32x4{0u, 0u, 0u, 0u};
     }
   }
-  block_sync();
-
-  if (tid < D) {
-    const int d = tid;
-    const float count = (float)n;
-    const int64_t o = (((int64_t)b * a.blocks + j) * a.kv_heads + g) * D + d;
-    if (DO_K) {
-      const float s = part[0][0][d] + part[0][1][d] + part[0][2][d] + part[0][3][d];
-      const float s2 = part[1][0][d] + part[1][1][d] + part[1][2][d] + part[1][3][d];
-      const float mean = s / count;
-      if (a.mean_k_bf16) a.mean_k_bf16[o] = to_bf16_bits(mean);
-      if (a.mean_k) a.mean_k[o] = mean;
-      if (a.var_k) a.var_k[o] = fmaxf(s2 / count - mean * mean, 0.0f);
-    }
-    if (DO_V) {
-      const float s = part[2][0][d] + part[2][1][d] + part[2][2][d] + part[2][3][d];
-      const float s2 = part[3][0][d] + part[3][1][d] + part[3][2][d] + part[3][3][d];
-      const float mean = s / count;
-      const float var = fmaxf(s2 / count - mean * mean, 0.0f);
-      if (a.mean_v) a.mean_v[o] = mean;
-      if (a.sigma_v) {
-        const float total = wave_sum(var);
-        if ((tid & 63) == 0) sig_part[tid >> 6] = total;
-      }
-    }
-  }
-  if (a.counts && blockIdx.y == 0 && tid == 0) a.counts[j] = n;
 
   if (DO_TILES) {
-    // Transposed write-out: thread -> (dim row d, 8-slot chunk gc); each gathers the
-    // 8 keys of its slots from the staged rows and stores 16 bytes at the swizzled
-    // chunk position (D = 128: [dim][128 slots], chunk gc ^ (d & 15); D = 256: sub-block
-    // gc / 4 of [dim][32 slots], chunk (gc & 3) ^ ((d >> 2) & 3)).
-    uint16_t* tile = a.value_tiles + tile_off;
-    const int my_half = rg * kRowsPer / (kBlock / 2);
+    if (!is_v) {
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      if (my_half == hh) {
+      for (int i = 0; i < kPoolRows; ++i) {
+        const int row = rg * kPoolRows + i;
+        *reinterpret_cast<u32x4*>(a.key_tiles + tile_off + row * D + ((c ^ i) << 3)) = raw[i];
+      }
+    } else {
+      // slot -> key inside the 16 rows: 4 * half + (m % 4) + 8 * (m / 4) for slot
+      // 8 * half + m; 16-byte chunk `chunk` of dim row d at the swizzled position
 #pragma unroll
-        for (int i = 0; i < kRowsPer; ++i) {
-          const int row = rg * kRowsPer + i - hh * (kBlock / 2);
-          uint32_t* dst = reinterpret_cast<uint32_t*>(vrows + row * kVPitch + c * 8);
+      for (int half = 0; half < 2; ++half) {
+        const int chunk = rg * 2 + half;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dst[e] = vraw[i][e];
+        for (int x = 0; x < 8; ++x) {
+          const int d = c * 8 + x;
+          u32x4 w;
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            const int key = 4 * half + 2 * (m & 1) + 8 * (m >> 1);
+            const uint32_t lo = raw[key][x >> 1], hi = raw[key + 1][x >> 1];
+            w[m] = (x & 1) ? high_halves(lo, hi) : low_halves(lo, hi);
+          }
+          uint16_t* dst =
+              D == 128 ? vtile + d * kBlock + ((chunk ^ (d & 15)) << 3)
+                       : vtile + (chunk >> 2) * (D * 32) + d * 32 + (((chunk & 3) ^ ((d >> 2) & 3)) << 3);
+          *reinterpret_cast<u32x4*>(dst) = w;
         }
       }
-      block_sync();
-#pragma unroll
-      for (int i = 0; i < 8 * D / kPoolThreads; ++i) {
-        const int id = tid + kPoolThreads * i;  // 0 .. 8 D - 1
-        const int d = id >> 3;                  // dim row of the tile
-        const int chunk = hh * 8 + (id & 7);    // slots chunk * 8 .. chunk * 8 + 7 (keys of this half)
-        uint32_t w[4];
-#pragma unroll
-        for (int m = 0; m < 8; m += 2) {
-          const int s0 = chunk * 8 + m;
-          // slot -> key: chunk16 * 16 + 4 * half + (m % 4) + 8 * (m / 4)
-          const int c16 = s0 >> 4, half = (s0 >> 3) & 1, mm = s0 & 7;
-          const int key0 = c16 * 16 + 4 * half + (mm & 3) + 8 * (mm >> 2) - hh * (kBlock / 2);
-          const uint32_t lo = vrows[key0 * kVPitch + d];
-          const uint32_t hi = vrows[(key0 + 1) * kVPitch + d];
-          w[m >> 1] = lo | (hi << 16);
-        }
-        uint16_t* dst;
-        if (D == 128)
-          dst = tile + d * kBlock + ((chunk ^ (d & 15)) << 3);
-        else
-          dst = tile + (chunk >> 2) * (D * 32) + d * 32 + (((chunk & 3) ^ ((d >> 2) & 3)) << 3);
-        *reinterpret_cast<u32x4*>(dst) = u32x4{w[0], w[1], w[2], w[3]};
-      }
-      if (hh == 0) block_sync();   // every read of the first half is done
     }
   }
-  if (DO_V) {
+  if ((DO_K && !is_v) || (DO_V && is_v)) column_sums<D>(raw, c, rg, lane, part);
+  if (a.counts && blockIdx.y == 0 && tid == 0) a.counts[j] = n;
+  block_sync();
+  if (DO_TILES) {   // all waves: whole lines of the value tile
+#pragma unroll
+    for (int i = 0; i < kBlock * D / 8 / (2 * D); ++i) {
+      const int e = (i * 2 * D + tid) * 8;
+      *reinterpret_cast<u32x4*>(a.value_tiles + tile_off + e) =
+          *reinterpret_cast<const u32x4*>(vtile + e);
+    }
+  }
+  if (!DO_K && !DO_V) return;
+
+  const float count = (float)n;
+  const int64_t o = (((int64_t)b * a.blocks + j) * a.kv_heads + g) * D + tx;
+  if (DO_K && !is_v) {
+    const float s = part[0][0][tx] + part[0][1][tx] + part[0][2][tx] + part[0][3][tx];
+    const float s2 = part[1][0][tx] + part[1][1][tx] + part[1][2][tx] + part[1][3][tx];
+    const float mean = s / count;
+    if (a.mean_k_bf16) a.mean_k_bf16[o] = to_bf16_bits(mean);
+    if (a.mean_k) a.mean_k[o] = mean;
+    if (a.var_k) a.var_k[o] = fmaxf(s2 / count - mean * mean, 0.0f);
+  }
+  if (DO_V && is_v) {
+    const float s = part[0][0][tx] + part[0][1][tx] + part[0][2][tx] + part[0][3][tx];
+    const float s2 = part[1][0][tx] + part[1][1][tx] + part[1][2][tx] + part[1][3][tx];
+    const float mean = s / count;
+    const float var = fmaxf(s2 / count - mean * mean, 0.0f);
+    if (a.mean_v) a.mean_v[o] = mean;
+    if (a.sigma_v) {
+      const float total = wave_sum(var);
+      if (lane == 0) part[0][0][tx] = total;
+    }
+  }
+  if (DO_V && a.sigma_v) {
     block_sync();
-    if (a.sigma_v && tid == 0) {
+    if (tid == 0) {
       float total = 0.0f;
 #pragma unroll
-      for (int x = 0; x < D / 64; ++x) total += sig_part[x];
+      for (int x = 0; x < D / 64; ++x) total += part_s[kReadK][0][0][64 * x];
       a.sigma_v[((int64_t)b * a.blocks + j) * a.kv_heads + g] = sqrtf(total);
     }
   }
@@ -212,14 +226,14 @@ using namespace spx;
 template <int D>
 static void launch_pool(int variant, dim3 grid, hipStream_t st, const PoolArgs& a) {
   switch (variant) {
-    case 0: pool_kernel<D, false, false, false><<<grid, kPoolThreads, 0, st>>>(a); break;
-    case 1: pool_kernel<D, false, false, true><<<grid, kPoolThreads, 0, st>>>(a); break;
-    case 2: pool_kernel<D, false, true, false><<<grid, kPoolThreads, 0, st>>>(a); break;
-    case 3: pool_kernel<D, false, true, true><<<grid, kPoolThreads, 0, st>>>(a); break;
-    case 4: pool_kernel<D, true, false, false><<<grid, kPoolThreads, 0, st>>>(a); break;
-    case 5: pool_kernel<D, true, false, true><<<grid, kPoolThreads, 0, st>>>(a); break;
-    case 6: pool_kernel<D, true, true, false><<<grid, kPoolThreads, 0, st>>>(a); break;
-    default: pool_kernel<D, true, true, true><<<grid, kPoolThreads, 0, st>>>(a); break;
+    case 0: pool_kernel<D, false, false, false><<<grid, D, 0, st>>>(a); break;
+    case 1: pool_kernel<D, false, false, true><<<grid, 2 * D, 0, st>>>(a); break;
+    case 2: pool_kernel<D, false, true, false><<<grid, D, 0, st>>>(a); break;
+    case 3: pool_kernel<D, false, true, true><<<grid, 2 * D, 0, st>>>(a); break;
+    case 4: pool_kernel<D, true, false, false><<<grid, D, 0, st>>>(a); break;
+    case 5: pool_kernel<D, true, false, true><<<grid, 2 * D, 0, st>>>(a); break;
+    case 6: pool_kernel<D, true, true, false><<<grid, 2 * D, 0, st>>>(a); break;
+    default: pool_kernel<D, true, true, true><<<grid, 2 * D, 0, st>>>(a); break;
   }
 }
 
