@@ -31,8 +31,11 @@
 //   * Full blocks are software-pipelined over their four 32-key sub-blocks (matrix
 //     work of one sub-block around the exponentials of the previous one); the
 //     running max moves lazily (only by more than 2^64), so the O rescale is a
-//     rarely taken wave-uniform branch. The diagonal blocks (t and t - 1) run last
-//     through a masked path in which wave w touches only key sub-blocks 0 .. w.
+//     rarely taken wave-uniform branch. Both tiles' diagonal blocks run last, side by
+//     side (tile t - 1's is still in LDS as tile t's last full block), through a masked
+//     path in which wave w touches only key sub-blocks 0 .. w of its tile. (One after
+//     the other, tile t taking block t - 1 through the masked path's unpipelined code:
+//     layers of 4 x 2113 tokens 223 -> 217 us, 4096 155 -> 152, 32640 6361 -> 6347.)
 //   * Grid order: (tile pair, q head) items heaviest-first. Workgroup i runs on XCD
 //     i % 8; a (batch, kv group) stream is served by a fixed set of XCDs, so the q
 //     heads sharing a KV block read it from the same L2s, and with 8 / (B * Hkv)
@@ -867,7 +870,9 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int item = w >> 2;                           // 0: tile t, 1: tile t - 1
-  const int wi = w & 3;                              // wave inside its item
+  // wave inside its item: rows 32 wi ..; waves w and w + 4 share a SIMD, and on the
+  // diagonal wave wi has wi + 1 sub-blocks, so the second item deals them in reverse
+  const int wi = (w & 3) ^ (item ? 3 : 0);
   const int col = lane & 31, half = lane >> 5;
   const int q_pos = wi * 32 + col;                   // this lane's query inside its tile
   const float scale = a.scale_log2;
@@ -932,9 +937,10 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
     for (int dc = 0; dc < 8; ++dc)
       ws.qb[dc] = as_bf16x8(*reinterpret_cast<const u32x4*>(qs + q_stage_chunk(q_pos, 2 * dc + half) * 8));
   }
-  // Processing order: every listed block except the two diagonal ones (t, t - 1),
-  // ascending, then the diagonal ones. The block loop for the first part has a
-  // single (unmasked) code path, which keeps O in one register set.
+  // Processing order: the unmasked blocks first (all but the tiles' own ones t and
+  // t - 1, ascending, then those two where the other tile lists them: t - 1 for tile t),
+  // through a block loop with a single (unmasked) code path, which keeps O in one
+  // register set; then both tiles' diagonal blocks side by side.
   auto times_listed = [&](int it, int j) {
     return (int)((mult[it][j >> 1] >> ((j & 1) * 16)) & 0xffffu);
   };
@@ -964,44 +970,39 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
     for (int x = 0; x < kAttnThreads / 64; ++x) nu += wave_counts[x];
     block_sync();
   }
-  const int n_full = __builtin_amdgcn_readfirstlane(nu);
-  // the diagonal blocks t - 1, t (known ids) go after the others, ascending
+  // t for tile t - 1 (never routed there), then t - 1 for tile t: the last unmasked
+  // block is then in LDS when tile t - 1 takes it as its diagonal. Entry n_full is the
+  // diagonal block t (its copy is issued with the others').
   if (tid == 0) {
     int n = nu;
 #pragma unroll
-    for (int i = 1; i >= 0; --i) {
+    for (int i = 0; i < 2; ++i) {
       const int j = t_item[i];
       if (j < 0) continue;
-      const int c0 = times_listed(0, j), c1 = times_listed(1, j);
-      for (int k = 0; k < max(c0, c1); ++k, ++n) {
+      for (int k = times_listed(1 - i, j); k > 0; --k, ++n) {
         ulist[n] = (int16_t)j;
-        uflag[n] = (uint8_t)((c0 > k ? 1 : 0) | (c1 > k ? 2 : 0));
+        uflag[n] = (uint8_t)(2 >> i);
       }
     }
+    ulist[n] = (int16_t)t_item[0];
     wave_counts[0] = n;
   }
   block_sync();
-  nu = __builtin_amdgcn_readfirstlane(wave_counts[0]);
-  if (EXACT && nu > 0) {
+  const int n_full = __builtin_amdgcn_readfirstlane(wave_counts[0]);
+  // diagonal block of each tile: times listed
+  const int n_diag0 = __builtin_amdgcn_readfirstlane(times_listed(0, t_item[0]));
+  const int n_diag1 =
+      t_item[1] < 0 ? 0 : __builtin_amdgcn_readfirstlane(times_listed(1, t_item[1]));
+  nu = n_full + (n_diag0 > 0 ? 1 : 0);   // blocks copied in the list's order
+  if (EXACT && (nu > 0 || n_diag1 > 0)) {
     const int64_t tile_elems = (int64_t)kBlock * kHeadDim;
     const uint16_t* kbase = a.kt + (((int64_t)b * a.kv_heads + g) * a.blocks) * tile_elems;
     const uint16_t* vbase = a.vt + (((int64_t)b * a.kv_heads + g) * a.blocks) * tile_elems;
-    {
+    if (nu > 0) {
       const int j0 = __builtin_amdgcn_readfirstlane(ulist[0]);
       dma_tile(kbase + j0 * tile_elems, kbuf[0], tid);
       dma_tile(vbase + j0 * tile_elems, vbuf[0], tid);
     }
-    // Publish block u (its copy was issued one step earlier) and start the copy of
-    // block u + 1 into the other buffers, where it lands during block u's math.
-    auto begin_block = [&](int u) {
-      wait_tiles();
-      block_sync();  // block u visible to all; every wave is done with block u - 1
-      if (u + 1 < nu) {
-        const int jn = __builtin_amdgcn_readfirstlane(ulist[u + 1]);
-        dma_tile(kbase + jn * tile_elems, kbuf[(u + 1) & 1], tid);
-        dma_tile(vbase + jn * tile_elems, vbuf[(u + 1) & 1], tid);
-      }
-    };
     const OperandTables tables = operand_tables(kbuf[0], vbuf[0]);
     int u = 0;
     bf16x8 rv[8], pend[2];  // the pending P V product of the last full block
@@ -1036,22 +1037,24 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
     }
     sub_pv(rv, pend, ws);
     if (ws.thr != -INFINITY) ws.m = -ws.neg_m;  // the max the full blocks settled on
-    u = n_full;
-    for (; u < nu; ++u) {
-      const int cur = u & 1;
-      const int j = __builtin_amdgcn_readfirstlane(ulist[u]);
-      const int f = __builtin_amdgcn_readfirstlane(uflag[u]);
-      begin_block(u);
-      if ((f >> item) & 1) {
-        if (j != t) {
-          exact_block<4, false>(kbuf[cur], vbuf[cur], ws, scale, q_pos);
-        } else {
-          switch (wi) {  // wave wi reaches key sub-blocks 0 .. wi of the diagonal block
-            case 0: exact_block<1, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-            case 1: exact_block<2, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-            case 2: exact_block<3, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-            default: exact_block<4, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-          }
+    // Diagonal blocks: t is in (or on its way to) buffer n_full & 1, t - 1 in the other
+    // one if it was the last unmasked block, else it is copied there now.
+    const int other = (n_full & 1) ^ 1;
+    if (n_diag1 > 0 && (n_full == 0 || ulist[n_full - 1] != t_item[1])) {
+      block_sync();   // every wave is done with the last unmasked block
+      dma_tile(kbase + t_item[1] * tile_elems, kbuf[other], tid);
+      dma_tile(vbase + t_item[1] * tile_elems, vbuf[other], tid);
+    }
+    wait_tiles();
+    block_sync();
+    {
+      const int cur = item ? other : n_full & 1;
+      for (int k = item ? n_diag1 : n_diag0; k > 0; --k) {
+        switch (wi) {  // wave wi reaches key sub-blocks 0 .. wi of the diagonal block
+          case 0: exact_block<1, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          case 1: exact_block<2, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          case 2: exact_block<3, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          default: exact_block<4, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
         }
       }
     }
@@ -1107,7 +1110,7 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
   const float inv = any ? 1.0f / l : 0.0f;
   const int tx = thread_x();
   const int half_e = (tx >> 5) & 1;
-  const int wq = (tx >> 6) & 3;                       // wave inside its item
+  const int wq = ((tx >> 6) & 3) ^ (tx >= kItemWaves * 64 ? 3 : 0);   // wave inside its item
   const int64_t qrow = (int64_t)t * kBlock + wq * 32 + (tx & 31);
   if (OUT_F32) {
     if (live && qrow < a.seq) {
