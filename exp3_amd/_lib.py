@@ -62,9 +62,10 @@ _PROTOTYPES = {
     "spx_decode_attention": [_P, _S, _P, _S, _P, _S, _I, _I, _I, _I, _I, _F, _P, _P, _P],
 }
 
-# helpers with other return types
+# helpers without a status: sizes (int64)
 _SIZE_FUNCTIONS = {"spx_selector_workspace_bytes": [_I, _I, _I, _I],
-                   "spx_decode_workspace_bytes": [_I, _I, _I, _I, _I]}
+                   "spx_decode_workspace_bytes": [_I, _I, _I, _I, _I],
+                   "spx_attention_queue_ints": [_I, _I, _I, _I, _I]}
 
 EXPORTED_SYMBOLS = tuple(_PROTOTYPES) + tuple(_SIZE_FUNCTIONS) + ("spx_last_error",
                                                                    "spx_abi_version")
@@ -134,6 +135,13 @@ def stream(device: torch.device) -> int:
     of the 12 to 60 us that a short call spends on the host)."""
     index = torch.cuda.current_device() if device.index is None else device.index
     return torch._C._cuda_getCurrentRawStream(index)
+
+
+def work_queue(batch, sequence, q_heads, kv_heads, head_dim, device):
+    """Zeroed work counters for an attention launch of this shape, or None where the
+    kernel runs faster without them."""
+    ints = load().spx_attention_queue_ints(batch, sequence, q_heads, kv_heads, head_dim)
+    return torch.zeros(ints, dtype=torch.int32, device=device) if ints else None
 
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:

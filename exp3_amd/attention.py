@@ -264,7 +264,7 @@ class AttentionBackend:
                        _lib.ptr(indices), _lib.strides(indices), _lib.ptr(counts),
                        _lib.strides(counts))
         # zeroed counters of the kernel's persistent grid (work items taken in turn)
-        queue = torch.zeros(_lib.WORK_QUEUE_INTS, dtype=torch.int32, device=device)
+        queue = _lib.work_queue(batch, sequence, q_heads, k.shape[2], head_dim, device)
         common_tail = (batch, sequence, q_heads, k.shape[2], head_dim, self.block_size,
                        float(scale), _lib.ptr(output), _lib.strides(output), _lib.ptr(lse),
                        _lib.strides(lse), _lib.ptr(queue), _lib.stream(device))

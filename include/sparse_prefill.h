@@ -194,8 +194,11 @@ int spx_selector_scores_noalloc(const void* q, const int64_t* q_strides, const f
  * XCDs take more of the light last third of the tile pairs); at head_dim 256 the
  * last third of the tiles is taken from work_queue[0] the same way. The values it
  * is left holding are unspecified: zero it before the next use, and use one array
- * per launch in flight. NULL keeps one workgroup per item; the results are
- * identical either way.
+ * per launch in flight. NULL keeps one workgroup per item: a tile pair, or (head_dim
+ * 128, short launches) a single tile. The results are identical either way for
+ * ascending lists; for others the blocks may be added in another order.
+ * spx_attention_queue_ints says which is faster for a shape: SPX_WORK_QUEUE_INTS, or 0
+ * for NULL.
  * Replaces upstream/flashprefill_native_forward.py:478-521 (exact_attention) and the
  * Triton kernel _flash_forward (:215-354). */
 int spx_exact_attention(const void* q, const int64_t* q_strides, const void* key_tiles,
@@ -206,6 +209,9 @@ int spx_exact_attention(const void* q, const int64_t* q_strides, const void* key
                         float scale, void* out, const int64_t* out_strides, float* lse,
                         const int64_t* lse_strides, int32_t* work_queue,
                         void* stream);
+
+/* The int32 count of the work queue to pass for this shape (0: pass NULL). */
+int64_t spx_attention_queue_ints(int batch, int seq, int q_heads, int kv_heads, int head_dim);
 
 /* Exact attention with the block-mean correction fused in: each row additionally
  * attends to the fp32 mean K / mean V (logit + ln n_j) of every full-history block

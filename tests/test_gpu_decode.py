@@ -5,8 +5,8 @@ steps) and several steps per workgroup; every head layout incl. more than 16 q h
 per KV head; cache slices and [B, S, H, D] views as inputs.
 
 Tolerance: fp32 scores and sums leave about 1e-6 of the largest value, the bf16 output
-2^-9 of its own: |got - want| <= 2^-8 |want| + 1e-4 admits both with room for a sum of
-fp32 rounding over 10^5 keys."""
+half a step, 2^-8 of its own: |got - want| <= 2^-8 |want| + 1e-4 admits both with room for
+a sum of fp32 rounding over 10^5 keys."""
 
 import pytest
 import torch
