@@ -120,14 +120,14 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
     return None if tensor is None else tensor.data_ptr()
 
 
-_STRIDES = tuple(ctypes.c_int64 * n for n in range(6))
+STRIDES = tuple(ctypes.c_int64 * n for n in range(6))
 
 
 def strides(tensor: torch.Tensor | None):
     if tensor is None:
         return None
     values = tensor.stride()
-    return _STRIDES[len(values)](*values)
+    return STRIDES[len(values)](*values)
 
 
 def stream(device: torch.device) -> int:

@@ -294,6 +294,101 @@ class AttentionBackend:
         _, _, tiles = self._pool(k, v, False, False, True)
         return self._attention(q, k, tiles, None, None, scale, None, want_lse=False)
 
+    def _prefill(self, q, k, v, scale):
+        """One prefill layer of any method as bare launches, nothing between the stages
+        but pointers: all intermediate buffers are parts of one allocation, and what the
+        method does not read (the selection mask of the V1 route, unused moments) is not
+        written. The stage functions above do the same launches through tensors, for
+        profiles, captures and callers of the stages; their dozen allocations and views
+        kept layers of up to 1100 tokens bound by the host (52 us of Python per layer,
+        28/4 heads; here 30)."""
+        method, block_size = self.method, self.block_size
+        batch, sequence, q_heads, head_dim = q.shape
+        kv_heads = k.shape[2]
+        blocks = _blocks(sequence, block_size)
+        device = q.device
+        stream = _lib.stream(device)
+        shape = (batch, sequence, q_heads, kv_heads, head_dim, block_size)
+        selector = method in kernels.SELECTORS
+        v1 = method in V1_ROUTED_METHODS
+        rescue = method in RESCUE_METHODS
+        size = 0
+
+        def take(nbytes):
+            nonlocal size
+            offset, size = size, size + ((nbytes + 255) & ~255)
+            return offset
+
+        vectors = batch * blocks * kv_heads * head_dim
+        entries = batch * blocks * blocks * q_heads
+        tile_bytes = 2 * vectors * block_size
+        key_tiles, value_tiles = take(tile_bytes), take(tile_bytes)
+        kbar = take(2 * vectors) if v1 else None
+        moments = method in MEAN_METHODS or method == "fp_v1_rescue_v2"
+        mean_k = mean_v = counts = var_k = sigma_v = None
+        if moments:
+            mean_k, mean_v, counts = take(4 * vectors), take(4 * vectors), take(4 * blocks)
+        if selector:
+            var_k, sigma_v = take(4 * vectors), take(4 * batch * blocks * kv_heads)
+            nbytes = _lib.load().spx_selector_workspace_bytes(batch, sequence, kv_heads, head_dim)
+            split = take(max(nbytes, 0))
+            scores, mask = take(4 * entries), take(entries)
+        if rescue:
+            qmean, choice = take(4 * batch * blocks * q_heads * head_dim), take(entries)
+        indices = list_counts = None
+        if method != "dense":
+            indices, list_counts = take(8 * entries), take(4 * batch * blocks * q_heads)
+        space = torch.empty(size, dtype=torch.uint8, device=device)
+        base = space.data_ptr()
+
+        def at(offset):
+            return None if offset is None else base + offset
+
+        four, three = _lib.STRIDES[4], _lib.STRIDES[3]
+        qs, ks, vs = _lib.strides(q), _lib.strides(k), _lib.strides(v)
+        qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
+        entry_strides = four(blocks * blocks * q_heads, blocks * q_heads, q_heads, 1)
+        rules = (int(self.sink_blocks), int(self.window_blocks), int(self.last_full_blocks))
+        _lib.call("spx_block_pool", kp, ks, vp, vs, batch, sequence, kv_heads, head_dim, block_size,
+                  at(kbar), at(mean_k), at(mean_v), at(var_k), at(sigma_v), at(counts),
+                  at(key_tiles), at(value_tiles), stream)
+        if v1:
+            _lib.call("spx_v1_route", qp, qs, at(kbar),
+                      four(blocks * kv_heads * head_dim, kv_heads * head_dim, head_dim, 1), *shape,
+                      scale, float(self.alpha), *rules, None, at(indices), at(list_counts), None,
+                      stream)
+        elif selector:
+            if nbytes < 0:
+                raise ValueError(
+                    f"selector_scores: unsupported shape {tuple(q.shape)} (head_dim 128 or 256)")
+            _lib.call("spx_selector_scores", qp, qs, at(mean_k), at(var_k), at(sigma_v), at(counts),
+                      *shape, _lib.SELECTOR_IDS[method], scale, at(split), at(scores),
+                      entry_strides, stream)
+            _lib.call("spx_protected_selection", at(scores), entry_strides, batch, blocks, blocks,
+                      q_heads, float(self.alpha), *rules, at(mask), at(indices), at(list_counts),
+                      stream)
+        if rescue:
+            _lib.call("spx_tile_mean_query", qp, qs, batch, sequence, q_heads, head_dim, block_size,
+                      at(qmean), stream)
+            _lib.call("spx_rescue_choice", at(qmean), at(key_tiles), *shape, at(choice), stream)
+        output = torch.empty(batch, sequence, q_heads, head_dim, dtype=q.dtype, device=device)
+        queue = _lib.work_queue(batch, sequence, q_heads, kv_heads, head_dim, device)
+        if head_dim in upstream._ATTENTION_CONFIGS:   # what attention_tile_sizes() reports
+            upstream._flash_forward.best_config = upstream._ATTENTION_CONFIGS[head_dim]
+        head = (qp, qs, at(key_tiles), at(value_tiles), at(indices),
+                entry_strides if indices is not None else None, at(list_counts),
+                three(blocks * q_heads, q_heads, 1) if indices is not None else None)
+        tail = (*shape, scale, output.data_ptr(), _lib.strides(output), None, None, _lib.ptr(queue),
+                stream)
+        if rescue:
+            _lib.call("spx_sparse_attention_rescue", *head, at(choice), vp, vs, at(mean_k),
+                      at(mean_v), int(moments), *tail)
+        elif moments:
+            _lib.call("spx_sparse_attention_mean", *head, at(mean_k), at(mean_v), at(counts), *tail)
+        else:
+            _lib.call("spx_exact_attention", *head, *tail)
+        return output
+
     @staticmethod
     def _decode(query, key, value, scale):
         """One query row per head against the whole cache -> [B, 1, Hq, D]."""
@@ -343,6 +438,12 @@ class AttentionBackend:
             ).transpose(1, 2).contiguous()
             if self.record and is_prefill:
                 record["accounting"] = self._dense_accounting(query)
+        elif (not self.record and self.capture_callback is None and self.kernel_events is None
+              and not (self.alpha == 0 and self.method in kernels.SELECTORS)):
+            _lib.require_gpu(query, key, value)
+            output = self._prefill(_lib.kernel_view(query.transpose(1, 2)),
+                                   _lib.kernel_view(key.transpose(1, 2)),
+                                   _lib.kernel_view(value.transpose(1, 2)), float(scaling))
         elif self.method == "dense":
             q = _lib.kernel_view(query.transpose(1, 2))
             k = _lib.kernel_view(key.transpose(1, 2))
