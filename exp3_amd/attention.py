@@ -68,6 +68,18 @@ def _blocks(sequence: int, block_size: int) -> int:
     return (sequence + block_size - 1) // block_size
 
 
+def _layer_shapes_match(query, key, value) -> bool:
+    """Whether K and V have the shape that Q implies. One set of sizes describes all
+    buffers of AttentionBackend._prefill; any other call takes the stage functions, which
+    size each buffer by its own tensor and refuse what does not fit."""
+    if query.dim() != 4 or key.shape != value.shape:
+        return False
+    batch, q_heads, sequence, head_dim = query.shape
+    kv_heads = key.shape[1]
+    return (0 not in query.shape and kv_heads > 0 and q_heads % kv_heads == 0
+            and tuple(key.shape) == (batch, kv_heads, sequence, head_dim))
+
+
 def _decode_kernel_takes(query, key, value, scaling) -> bool:
     """Whether a non-prefill call is a decode step of spx_decode_attention: one query
     row per head of plain bf16 GPU tensors in a layout it reads in place, and nothing
@@ -439,7 +451,8 @@ class AttentionBackend:
             if self.record and is_prefill:
                 record["accounting"] = self._dense_accounting(query)
         elif (not self.record and self.capture_callback is None and self.kernel_events is None
-              and not (self.alpha == 0 and self.method in kernels.SELECTORS)):
+              and not (self.alpha == 0 and self.method in kernels.SELECTORS)
+              and _layer_shapes_match(query, key, value)):
             _lib.require_gpu(query, key, value)
             output = self._prefill(_lib.kernel_view(query.transpose(1, 2)),
                                    _lib.kernel_view(key.transpose(1, 2)),

@@ -50,3 +50,20 @@ def test_entry_point_validation():
     assert size(1, 256, 16, 4, 256) == 0 and size(2, 257, 16, 4, 256) == 3 * 32 * 258 * 4
     assert size(1, 131072, 28, 4, 128) == 256 * 28 * 130 * 4
     assert size(1, 512, 28, 4, 64) == size(0, 512, 28, 4, 128) == -1
+
+
+def test_prefill_scratch_needs_matching_shapes():
+    """Calls whose Q, K and V disagree stay with the stage functions and their checks."""
+    def x(*shape):
+        return torch.empty(*shape)
+
+    def match(*shapes):
+        return attention._layer_shapes_match(*(x(*s) for s in shapes))
+
+    q, kv = (2, 8, 300, 128), (2, 4, 300, 128)
+    assert match(q, kv, kv)
+    for bad in ((1, 4, 300, 128), (2, 3, 300, 128), (2, 0, 300, 128), (2, 4, 300, 256),
+                (2, 4, 299, 128), (4, 300, 128)):
+        assert not match(q, bad, bad) and not match(q, kv, bad) and not match(q, bad, kv)
+    assert not match((0, 8, 300, 128), (0, 4, 300, 128), (0, 4, 300, 128))
+    assert not match(q[1:], kv, kv)

@@ -54,3 +54,15 @@ def test_refusals(gpu):
         backend.configure(method)
         with pytest.raises(ValueError):
             backend.forward(_Layer(), *(x[..., :cut].transpose(1, 2) for x in (q, k, v)), None, 0.1)
+
+
+@pytest.mark.parametrize("q_cut,k_cut", (((0, 1), (0, 2)), ((0, 2), (0, 1)), ((1, 3), (1, 2))))
+def test_mismatched_keys_reach_the_stage_checks(gpu, q_cut, k_cut):
+    """A selector layer whose Q and K differ in batch or do not divide in heads."""
+    q, k, v, _ = synthetic.make_inputs(300, seed=2, q_heads=4, kv_heads=2, batch=2, device="cuda")
+    q, k, v = (x.transpose(1, 2) for x in (q, k, v))
+    backend = attention.AttentionBackend(alpha=0.1, register=False)
+    backend.configure("cgf_mean", 0.1)
+    cut = lambda x, c: x.narrow(c[0], 0, c[1])    # noqa: E731
+    with pytest.raises(ValueError, match="does not match"):
+        backend.forward(_Layer(), cut(q, q_cut), cut(k, k_cut), cut(v, k_cut), None, 0.1)
