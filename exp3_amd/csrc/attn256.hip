@@ -5,7 +5,7 @@
 //
 // gfx950 mapping
 //   * One workgroup per (query tile t, q head h): four waves of 32 query rows, one
-//     wave per SIMD. A wave keeps its Q rows in registers as MFMA B operands (16
+//     wave per SIMD, two workgroups per CU. A wave keeps its Q rows in registers as MFMA B operands (16
 //     k-steps of 16 dims) and O^T (256 dims x 32 queries, eight 32 x 32 tiles) in
 //     the accumulators.
 //   * Keys stream in 32-key sub-blocks: the K rows (16 KB) and V^T (256 dims x 32
@@ -18,6 +18,12 @@
 //     layout of O^T += V^T P^T (key slot permutation of the value tiles). The running
 //     max moves only when a column's shifted score x = s * scale - m exceeds 2^64
 //     (lazy rescale); the common path checks each lane half's own max of x.
+//   * Short launches (G = 2) put two such groups of four waves on a tile: group g takes
+//     sub-blocks g, g + 2, ... with buffers of its own, one workgroup per CU, and the two
+//     groups' (max, sum, O) merge through the K / V buffers at the end, each group
+//     storing half of the dims. A workgroup of one group is a serial chain of up to 4 NB
+//     sub-blocks (the last tiles list every block), and with few items per CU the launch
+//     lasts as long as that chain, not as its work.
 //   * The tile's list (entries outside [0, NB) skipped, as the reference's loop
 //     never reads them usefully) is compacted into LDS once; as in the reference,
 //     only the diagonal block j == t is masked (key > query).
@@ -212,8 +218,94 @@ __device__ __forceinline__ void dma_16k(const uint16_t* src, uint16_t* lds, int 
   }
 }
 
-template <bool EXACT, bool TAIL, bool OUT_F32>
-__global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
+// Exchange slot i (< 8) of 16 KB: the four K buffers, then the four V buffers.
+__device__ __forceinline__ uint16_t* exchange_slot(uint16_t* k0, uint16_t* v0, int i) {
+  return i < 4 ? k0 + i * kSubElems : v0 + (i - 4) * kSubElems;
+}
+
+// O tiles FIRST .. FIRST + 3 of this lane to a slot.
+template <int FIRST>
+__device__ __forceinline__ void give_dims(const f32x16 (&o)[8], uint16_t* slot, int lane) {
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+      *reinterpret_cast<f32x4*>(slot + ((dt * 4 + x) * 64 + lane) * 8) =
+          f32x4{o[FIRST + dt][4 * x], o[FIRST + dt][4 * x + 1], o[FIRST + dt][4 * x + 2],
+                o[FIRST + dt][4 * x + 3]};
+}
+
+// O tiles FIRST .. FIRST + 3: own times its weight plus the slot's times the other's.
+template <int FIRST>
+__device__ __forceinline__ void take_dims(f32x16 (&o)[8], const uint16_t* slot, int lane,
+                                          float w_own, float w_other) {
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const f32x4 p = *reinterpret_cast<const f32x4*>(slot + ((dt * 4 + x) * 64 + lane) * 8);
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+        o[FIRST + dt][4 * x + y] = o[FIRST + dt][4 * x + y] * w_own + p[y] * w_other;
+    }
+}
+
+// O tiles FIRST .. FIRST + N - 1 (32 dims each) of a wave's 32 query rows, divided by l.
+// bf16: each lane holds 4-dim pieces of its query row, so stored directly every store
+// instruction would write 16 bytes into each of 32 rows. The wave stages its rows in
+// `stage` (free K / V buffer of its own, 16-byte chunk c of row r at c ^ (r % chunks)) and
+// stores whole row parts, 4 N lanes per row.
+template <bool OUT_F32, int FIRST, int N>
+__device__ __forceinline__ void store_rows(const Attn256Args& a, const f32x16 (&o)[8], float l,
+                                           int b, int t, int h, uint16_t* stage, int wv) {
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  // lane values re-derived here, so that nothing computed from them is hoisted above the
+  // block loops and held there
+  const int lane = opaque((int)threadIdx.x) & 63;
+  const int col = lane & 31, half = lane >> 5;
+  const int64_t row0 = (int64_t)t * kBlock + wv * 32;
+  if constexpr (OUT_F32) {
+    if (row0 + col < a.seq) {
+      float* dst =
+          static_cast<float*>(a.out) + b * a.os_b + (row0 + col) * a.os_s + h * a.os_h + 4 * half;
+#pragma unroll
+      for (int dt = FIRST; dt < FIRST + N; ++dt)
+#pragma unroll
+        for (int grp = 0; grp < 4; ++grp) {
+          const int r = 4 * grp;
+          *reinterpret_cast<f32x4*>(dst + dt * 32 + 8 * grp) =
+              f32x4{o[dt][r] * inv, o[dt][r + 1] * inv, o[dt][r + 2] * inv, o[dt][r + 3] * inv};
+        }
+    }
+  } else {
+    constexpr int kChunks = 4 * N, kRows = 64 / kChunks;   // chunks per row part, rows per store
+#pragma unroll
+    for (int dt = 0; dt < N; ++dt)
+#pragma unroll
+      for (int grp = 0; grp < 4; ++grp) {
+        const int r = 4 * grp;
+        u32x2 v;
+        v[0] = pack_bf16x2(o[FIRST + dt][r] * inv, o[FIRST + dt][r + 1] * inv);
+        v[1] = pack_bf16x2(o[FIRST + dt][r + 2] * inv, o[FIRST + dt][r + 3] * inv);
+        const int c = (dt * 4 + grp) ^ (col & (kChunks - 1));
+        *reinterpret_cast<u32x2*>(stage + (col * kChunks + c) * 8 + 4 * half) = v;
+      }
+    const int c = lane & (kChunks - 1);
+#pragma unroll
+    for (int i = 0; i < 32 / kRows; ++i) {
+      const int r = kRows * i + lane / kChunks;
+      const u32x4 v4 = *reinterpret_cast<const u32x4*>(
+          stage + (r * kChunks + (c ^ (r & (kChunks - 1)))) * 8);
+      if (row0 + r < a.seq)   // non-temporal: not read again here (keeps the K/V sub-blocks in L2)
+        __builtin_nontemporal_store(
+            v4, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(a.out) + b * a.os_b +
+                                         (row0 + r) * a.os_s + h * a.os_h + FIRST * 32 + c * 8));
+    }
+  }
+}
+
+template <bool EXACT, bool TAIL, bool OUT_F32, int G>
+__global__ __launch_bounds__(G * kA2Threads, 1) void attn256_kernel(Attn256Args a) {
   const int per_tile = a.batch * a.q_heads;
   int rank = (int)(blockIdx.x / per_tile), bh = (int)(blockIdx.x % per_tile);
   if (a.queue && rank >= a.static_ranks) {
@@ -231,24 +323,30 @@ __global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
   const int t = a.blocks - 1 - rank;  // heaviest tiles first
   const int b = bh / a.q_heads, h = bh % a.q_heads;
   const int g = h / (a.q_heads / a.kv_heads);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  // group of four waves, and thread and wave within it
+  const int grp = G > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kA2Threads) : 0;
+  const int tid = G > 1 ? (int)threadIdx.x % kA2Threads : (int)threadIdx.x;
+  const int lane = tid & 63, w = tid >> 6;
   const int col = lane & 31, half = lane >> 5;
 
-  __shared__ __align__(16) uint16_t kbuf[2][kSubElems];
-  __shared__ __align__(16) uint16_t vbuf[2][kSubElems];
+  // buffer pairs 2 grp and 2 grp + 1 are the group's
+  __shared__ __align__(16) uint16_t kbuf[2 * G][kSubElems];
+  __shared__ __align__(16) uint16_t vbuf[2 * G][kSubElems];
+  uint16_t(*const kb)[kSubElems] = kbuf + 2 * grp;
+  uint16_t(*const vb)[kSubElems] = vbuf + 2 * grp;
   __shared__ int list[kA2MaxBlocks];
   __shared__ int list_len;
   __shared__ uint32_t listed[TAIL ? kA2MaxBlocks / 32 : 1];   // membership of the tile's list
   __shared__ int16_t tlist[TAIL ? kA2MaxBlocks : 1];          // unlisted history blocks
-  __shared__ float tail_bias[kSub];
+  __shared__ float tail_bias[G][kSub];
   __shared__ int tail_len;
 
   if (TAIL) {
-    if (tid < kA2MaxBlocks / 32) listed[tid] = 0u;
+    if (threadIdx.x < kA2MaxBlocks / 32) listed[threadIdx.x] = 0u;
     block_sync();
   }
   // compacted block list: ids in [0, NB), list order
-  if (w == 0) {
+  if (grp == 0 && w == 0) {
     int n = a.idx ? a.cnt[b * a.cs_b + t * a.cs_t + h * a.cs_h] : t + 1;
     n = max(0, min(n, a.blocks));
     int base = 0;
@@ -268,16 +366,16 @@ __global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
     if (lane == 0) list_len = base;
   }
   block_sync();
-  const int steps = EXACT ? list_len * 4 : 0;
+  const int steps = EXACT ? list_len * 4 : 0;   // group grp takes grp, grp + G, ...
   const int64_t kv_block0 = ((int64_t)b * a.kv_heads + g) * a.blocks;
 
   auto issue = [&](int s, int buf) {
     const int j = __builtin_amdgcn_readfirstlane(list[s >> 2]);
     const int sb = s & 3;
-    dma_16k(a.kt + ((kv_block0 + j) * kBlock + sb * kSub) * kD2, kbuf[buf], tid);
-    dma_16k(a.vt + (kv_block0 + j) * (kBlock * kD2) + sb * kSubElems, vbuf[buf], tid);
+    dma_16k(a.kt + ((kv_block0 + j) * kBlock + sb * kSub) * kD2, kb[buf], tid);
+    dma_16k(a.vt + (kv_block0 + j) * (kBlock * kD2) + sb * kSubElems, vb[buf], tid);
   };
-  if (steps > 0) issue(0, 0);
+  if (steps > 0) issue(grp, 0);
 
   const int qr = w * 32 + col;  // query row within the tile
   const int64_t qrow = (int64_t)t * kBlock + qr;
@@ -305,14 +403,15 @@ __global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
   float thr = -INFINITY;     // lazy-move threshold on shifted scores (-inf before the max is set)
   float l = 0.0f;            // this half's share of the probability sum
 
-  for (int s = 0; s < steps; ++s) {
+  for (int it = 0; it < steps / G; ++it) {
+    const int s = it * G + grp;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    block_sync();  // sub-block s landed everywhere; buffers (s + 1) & 1 are free
-    if (s + 1 < steps) issue(s + 1, (s + 1) & 1);
+    block_sync();  // sub-block s landed everywhere; buffers (it + 1) & 1 are free
+    if (s + G < steps) issue(s + G, (it + 1) & 1);
     const int j = __builtin_amdgcn_readfirstlane(list[s >> 2]);
     const int sb = s & 3;
     f32x16 sc = {};
-    key_products(kbuf[s & 1] + col * kD2, e0, qb, sc);
+    key_products(kb[it & 1] + col * kD2, e0, qb, sc);
     // x = s * scale - m (diagonal block: keys above the query at -inf); the lazy
     // max check runs on x, per lane half, and forms the column max over both
     // halves only in the rare branch where some lane exceeds its threshold
@@ -324,12 +423,12 @@ __global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
       for (int r = 0; r < 16; ++r)
         if (sb * kSub + mfma32_row(r, lane) > qr) x[r] = -INFINITY;
     }
-    softmax_pv(x, vbuf[s & 1], o, neg_m, thr, l);
+    softmax_pv(x, vb[it & 1], o, neg_m, thr, l);
   }
 
   if constexpr (TAIL) {
     // the tail: history blocks j < t the tile does not list, ascending
-    if (w == 0) {
+    if (grp == 0 && w == 0) {
       int base = 0;
       for (int j0 = 0; j0 < t; j0 += 64) {
         const int j = j0 + lane;
@@ -344,16 +443,17 @@ __global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
     const int ntail = tail_len;
     const int epb = a.tail_kind == 2 ? 2 : 1;  // entries per unlisted block
     const int per_sub = kSub / epb;
-    for (int t0 = 0; t0 < ntail; t0 += per_sub) {
+    for (int t0 = 0; t0 < ntail; t0 += G * per_sub) {
       if (t0 > 0) block_sync();  // every wave is done with the previous tail sub-block
-      // one work item per (entry, 8-dim chunk): 32 x 32 over the four waves. Not
+      // each group its own 32 entries (past the last one: logit -inf), one work item
+      // per (entry, 8-dim chunk): 32 x 32 over the four waves. Not
       // unrolled: with O (128) and Q (64) live, four items' temporaries at once
       // would push the wave past 256 registers (AGPR spills, one wave per SIMD)
 #pragma unroll 1
       for (int k4 = 0; k4 < (kSub * (kD2 / 8)) / kA2Threads; ++k4) {
         const int e = opaque(tid) + k4 * kA2Threads;
         const int i = e >> 5, c = e & 31;
-        const int blk = t0 + i / epb, kind = i % epb;
+        const int blk = t0 + grp * per_sub + i / epb, kind = i % epb;
         const int j = blk < ntail ? (int)tlist[blk] : -1;
         float mk[8] = {}, mv[8] = {};
         float bi = -INFINITY;
@@ -395,78 +495,81 @@ __global__ __launch_bounds__(kA2Threads, 1) void attn256_kernel(Attn256Args a) {
             }
           }
         }
-        write_tail_entry256(kbuf[0], kbuf[1], vbuf[0], i, c, mk, mv);
-        if (c == 0) tail_bias[i] = bi;
+        write_tail_entry256(kb[0], kb[1], vb[0], i, c, mk, mv);
+        if (c == 0) tail_bias[grp][i] = bi;
       }
       block_sync();
       const int lane_t = opaque(lane);
       const int col_t = lane_t & 31;
       const int e0_t = (((col_t >> 1) & 7) << 4) + (((lane_t >> 5) ^ (col_t & 1)) << 3);
       f32x16 sc = {};
-      key_products(kbuf[0] + col_t * kD2, e0_t, qb, sc);   // hi rows
-      key_products(kbuf[1] + col_t * kD2, e0_t, qb, sc);   // lo rows
+      key_products(kb[0] + col_t * kD2, e0_t, qb, sc);   // hi rows
+      key_products(kb[1] + col_t * kD2, e0_t, qb, sc);   // lo rows
       f32x16 x;
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        x[r] = fmaf(sc[r], a.scale_log2, tail_bias[mfma32_row(r, lane_t)]) + neg_m;
-      softmax_pv(x, vbuf[0], o, neg_m, thr, l);
+        x[r] = fmaf(sc[r], a.scale_log2, tail_bias[grp][mfma32_row(r, lane_t)]) + neg_m;
+      softmax_pv(x, vb[0], o, neg_m, thr, l);
     }
   }
 
   l += __shfl_xor(l, 32);
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  if (OUT_F32) {
-    if (row_ok) {
-      float* dst = static_cast<float*>(a.out) + b * a.os_b + qrow * a.os_s + h * a.os_h + 4 * half;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) {
-#pragma unroll
-        for (int grp = 0; grp < 4; ++grp) {
-          const int r = 4 * grp;
-          *reinterpret_cast<f32x4*>(dst + dt * 32 + 8 * grp) =
-              f32x4{o[dt][r] * inv, o[dt][r + 1] * inv, o[dt][r + 2] * inv, o[dt][r + 3] * inv};
-        }
-      }
+  if constexpr (G == 2) {
+    // Both groups hold (max, sum, O) of the same rows over their own keys. Each hands the
+    // half of the dims that the other one stores over through the K / V buffers (16 KB a
+    // wave, 16-byte pieces in lane order) and merges its own half.
+    __shared__ float part_m[2][kBlock], part_l[2][kBlock];
+    const float own_m = thr == -INFINITY ? -INFINITY : -neg_m;
+    block_sync();   // every wave is done with the K / V buffers
+    const int mine = opaque((int)threadIdx.x);
+    const int ml = mine & 63, mw = __builtin_amdgcn_readfirstlane((mine >> 6) & 3);
+    const int row = mw * 32 + (ml & 31);
+    if (ml < 32) {
+      part_m[grp][row] = own_m;
+      part_l[grp][row] = l;
+    }
+    if (grp == 0) give_dims<4>(o, exchange_slot(kbuf[0], vbuf[0], 4 + mw), ml);
+    else give_dims<0>(o, exchange_slot(kbuf[0], vbuf[0], mw), ml);
+    block_sync();
+    const float other_m = part_m[1 - grp][row];
+    const float top = fmaxf(own_m, other_m);
+    const float w_own = own_m == -INFINITY ? 0.0f : exp2_fast(own_m - top);
+    const float w_other = other_m == -INFINITY ? 0.0f : exp2_fast(other_m - top);
+    // the two sums in the same order in both groups
+    const float l0 = grp == 0 ? l * w_own : part_l[0][row] * w_other;
+    const float l1 = grp == 0 ? part_l[1][row] * w_other : l * w_own;
+    l = l0 + l1;
+    neg_m = top == -INFINITY ? 0.0f : -top;
+    if (grp == 0) {
+      take_dims<0>(o, exchange_slot(kbuf[0], vbuf[0], mw), ml, w_own, w_other);
+      store_rows<OUT_F32, 0, 4>(a, o, l, b, t, h, kbuf[mw], mw);
+    } else {
+      take_dims<4>(o, exchange_slot(kbuf[0], vbuf[0], 4 + mw), ml, w_own, w_other);
+      store_rows<OUT_F32, 4, 4>(a, o, l, b, t, h, vbuf[mw], mw);
     }
   } else {
-    // Each lane holds 4-dim pieces of its query row, so stored directly every store
-    // instruction would write 16 bytes into each of 32 rows. The wave stages its
-    // 32 x 256 bf16 rows in one of the (now free) K / V buffers, 16-byte chunk c of
-    // row r at c ^ (r & 31), and stores whole 512-byte rows, 32 lanes per row.
     block_sync();   // every wave is done with the K / V buffers
-    // lane values re-derived here, so that nothing computed from them is hoisted
-    // above the block loops and held there
-    const int tx = opaque((int)threadIdx.x);
-    const int wv = __builtin_amdgcn_readfirstlane(tx >> 6);
-    const int lane_e = tx & 63, col_e = tx & 31, half_e = (tx >> 5) & 1;
-    uint16_t* stage = wv < 2 ? kbuf[wv] : vbuf[wv - 2];
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-#pragma unroll
-      for (int grp = 0; grp < 4; ++grp) {
-        const int r = 4 * grp;
-        u32x2 v;
-        v[0] = pack_bf16x2(o[dt][r] * inv, o[dt][r + 1] * inv);
-        v[1] = pack_bf16x2(o[dt][r + 2] * inv, o[dt][r + 3] * inv);
-        const int c = dt * 4 + grp;
-        *reinterpret_cast<u32x2*>(stage + col_e * kD2 + ((c ^ col_e) << 3) + 4 * half_e) = v;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = 2 * i + (lane_e >> 5), c = lane_e & 31;
-      const u32x4 v4 = *reinterpret_cast<const u32x4*>(stage + r * kD2 + ((c ^ r) << 3));
-      const int64_t row = (int64_t)t * kBlock + wv * 32 + r;
-      if (row < a.seq)   // non-temporal: not read again here (keeps the K/V sub-blocks in L2)
-        __builtin_nontemporal_store(
-            v4, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(a.out) + b * a.os_b + row * a.os_s +
-                                         h * a.os_h + c * 8));
-    }
+    const int mw = __builtin_amdgcn_readfirstlane(opaque((int)threadIdx.x) >> 6);
+    store_rows<OUT_F32, 0, 8>(a, o, l, b, t, h, mw < 2 ? kbuf[mw] : vbuf[mw - 2], mw);
   }
-  if (row_ok && a.lse && half == 0)
+  if (row_ok && a.lse && half == 0 && grp == 0)
     a.lse[b * a.ls_b + qrow * a.ls_s + h * a.ls_h] =
         l > 0.0f ? (log2f(l) - neg_m) * kLn2 : -INFINITY;
 }
+
+// Launches of up to kGroupItems items, or kGroupItemsLong of at least kGroupBlocksLong
+// blocks, use two groups per tile. There the chain of the longest list decides; with
+// more items the work does, and two groups, which meet at a barrier every sub-block and
+// leave a CU one workgroup (nothing beside its lists, Q and output), lose. Layers, one ->
+// two groups, 16/4 heads: every block listed, 2900 tokens (368 items) 140 -> 106 us, 4100
+// (528) 201 -> 172, 5000 (640) 251 -> 240, 8192 (1024) 547 -> 527; 4 x 700 (384) 67 -> 61;
+// routed, 1100 (144) 67 -> 60, 4500 (576) 196 -> 141, 6113 with rescue tokens (768) 289 ->
+// 225; 12/2 heads, 9000 (852) 357 -> 251. Beyond: 4 x 1300 (704, 11 blocks) 100 -> 116,
+// 4 x 2900 (1472) 253 -> 296, 12001 with every block (1504) 1040 -> 1089, routed 518 -> 417,
+// which the host cannot tell apart, 16000 dense (2000) 1771 -> 1845.
+constexpr int64_t kGroupItems = 384;
+constexpr int64_t kGroupItemsLong = 1024;
+constexpr int kGroupBlocksLong = 32;
 
 int launch_attention_256(const Attn256Options& opt, const void* q, const int64_t* q_strides,
                          const void* key_tiles, const void* value_tiles, const int64_t* indices,
@@ -514,9 +617,20 @@ int launch_attention_256(const Attn256Options& opt, const void* q, const int64_t
     grid = (unsigned)(a.static_ranks * batch * q_heads) + (unsigned)((a.dyn_items * 5 + 3) / 4);
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (opt.exact && !opt.tail) attn256_kernel<true, false, false><<<grid, kA2Threads, 0, st>>>(a);
-  else if (opt.exact) attn256_kernel<true, true, false><<<grid, kA2Threads, 0, st>>>(a);
-  else attn256_kernel<false, true, true><<<grid, kA2Threads, 0, st>>>(a);
+  const int64_t items = (int64_t)blocks * batch * q_heads;
+  const bool groups =
+      items <= kGroupItems || (items <= kGroupItemsLong && blocks >= kGroupBlocksLong);
+  const int T = (groups ? 2 : 1) * kA2Threads;
+  if (opt.exact && !opt.tail) {
+    if (groups) attn256_kernel<true, false, false, 2><<<grid, T, 0, st>>>(a);
+    else attn256_kernel<true, false, false, 1><<<grid, T, 0, st>>>(a);
+  } else if (opt.exact) {
+    if (groups) attn256_kernel<true, true, false, 2><<<grid, T, 0, st>>>(a);
+    else attn256_kernel<true, true, false, 1><<<grid, T, 0, st>>>(a);
+  } else {
+    if (groups) attn256_kernel<false, true, true, 2><<<grid, T, 0, st>>>(a);
+    else attn256_kernel<false, true, true, 1><<<grid, T, 0, st>>>(a);
+  }
   return launch_status("attention_d256");
 }
 

@@ -1,0 +1,73 @@
+"""Head dim 256: short launches split each tile's keys over two groups of waves
+(csrc/attn256.hip), long ones do not. The same sequence alone and within a batch that
+makes the launch long: same lists, outputs and LSEs within the rounding of the
+probabilities, for one to four blocks, ragged ends, empty, unsorted and repeated lists
+with entries outside the sequence, and every method's tail."""
+
+import pytest
+import torch
+
+from exp3_amd import attention, synthetic
+from exp3_amd.upstream import flashprefill_native_forward as upstream
+
+pytestmark = pytest.mark.gpu
+
+HEADS, KV, DIM = 16, 4, 256
+LONG = 1536 // HEADS + 1          # batch from which any launch is long
+
+
+def _inputs(length, seed):
+    q, k, v, _ = synthetic.make_inputs(length, seed=seed, q_heads=HEADS, kv_heads=KV, head_dim=DIM,
+                                       device="cuda")
+    return ((q.float() * 4).bfloat16(), (k.float() * 4).bfloat16(), v)
+
+
+def _batch(x):
+    return x.expand(LONG, *x.shape[1:]).contiguous()
+
+
+def _assert_close(got, want, v):
+    # bf16 keeps 8 significant bits: a rounding moves a value by up to 2^-8 of it. In each
+    # kernel P rounds against another running maximum (2^-8 of every key's share of the
+    # output, at most 2^-8 max |v|), then the output: both sides, twice
+    bound = 2 ** -7 * (v.float().abs().amax() + want.float().abs())
+    assert ((got.float() - want.float()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("length", (1, 31, 128, 129, 300, 512))
+def test_lists(gpu, length):
+    q, k, v = _inputs(length, 3 + length)
+    blocks = (length + 127) // 128
+    gen = torch.Generator().manual_seed(length)
+    # ids -1 and NB are dropped; a list may hold a block twice or none
+    idx = torch.randint(-1, blocks + 1, (1, blocks, blocks, HEADS), generator=gen)
+    tile = torch.arange(blocks)[None, :, None, None]
+    idx = torch.where((idx > tile) & (idx < blocks), tile, idx).cuda()
+    cnt = torch.randint(0, blocks + 1, (1, blocks, HEADS), generator=gen, dtype=torch.int32)
+    cnt[:, 0, 0] = 0
+    cnt = cnt.cuda()
+    out, lse = upstream.exact_attention(q, k, v, idx, cnt, DIM ** -0.5)
+    many, many_lse = upstream.exact_attention(*(_batch(x) for x in (q, k, v, idx, cnt)), DIM ** -0.5)
+    assert torch.equal(many[0], many[-1]) and not torch.isnan(out).any()
+    _assert_close(out[0], many[-1], v)
+    empty = torch.isinf(many_lse[-1])
+    assert torch.equal(torch.isinf(lse[0]), empty) and not out[0][empty].any()
+    # fp32 sums and base-2 logits of up to some 2^8
+    assert torch.allclose(lse[0][~empty], many_lse[-1][~empty], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("method", attention.METHODS)
+@pytest.mark.parametrize("length", (1, 260, 1089))
+def test_layers(gpu, method, length):
+    q, k, v = _inputs(length, 5)
+    backend = attention.AttentionBackend(alpha=0.6, register=False, dense_impl="hip", sink_blocks=1,
+                                         window_blocks=1, last_full_blocks=0)
+    backend.configure(method, 0.6)
+
+    class Layer:
+        layer_idx = 0
+
+    args = [x.transpose(1, 2) for x in (q, k, v)]
+    out, _ = backend.forward(Layer(), *args, None, DIM ** -0.5)
+    many, _ = backend.forward(Layer(), *(_batch(x) for x in args), None, DIM ** -0.5)
+    _assert_close(out[0], many[-1], v)

@@ -39,7 +39,7 @@ def test_against_64_bits(gpu, dim, batch, length, heads, layout):
     we, wm = (torch.exp(x.double() - want_lse)[..., None] for x in (el, ml))
     parts = (we * exact.double()).abs() + (wm * mean.double()).abs()
     want = we * exact.double() + wm * mean.double()
-    # bf16 rounding (2^-9 of the value) and fp32 weights: LSEs of up to 200 in 2^-24
+    # bf16 rounding (2^-8 of the value) and fp32 weights: LSEs of up to 200 in 2^-24
     # steps, so exp(le - total) is good to about 3e-5 of each part
     assert ((out.double() - want).abs() <= 2 ** -8 * want.abs() + 5e-5 * parts).all()
     assert torch.allclose(lse.double(), want_lse, rtol=1e-6, atol=1e-6)
