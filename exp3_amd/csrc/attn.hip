@@ -569,6 +569,9 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
   __shared__ uint32_t mult[2][kMaxBlocksAttn / 2];   // per-item times listed, 16 bits per block
   __shared__ float tail_bias[2][kTailTile];
   __shared__ int wave_counts[kAttnThreads / 64];
+  // of its own: with both lists empty no barrier separates its reads from the tail
+  // lists' writes to wave_counts
+  __shared__ int unmasked;
 
   const int tid = thread_x();
   const int lane = tid & 63;
@@ -689,10 +692,10 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
       }
     }
     ulist[n] = (int16_t)t_item[0];
-    wave_counts[0] = n;
+    unmasked = n;
   }
   block_sync();
-  const int n_full = __builtin_amdgcn_readfirstlane(wave_counts[0]);
+  const int n_full = __builtin_amdgcn_readfirstlane(unmasked);
   // diagonal block of each tile: times listed
   const int n_diag0 = __builtin_amdgcn_readfirstlane(times_listed(0, t_item[0]));
   const int n_diag1 =
