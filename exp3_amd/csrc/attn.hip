@@ -563,8 +563,9 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
   __shared__ __align__(16) uint16_t vbuf[2][kBlock * kBlock];
   // union of both lists, ascending; a block listed n times for an item appears
   // max over the items of n times, occurrence k flagged for the items listing it
-  // more than k times (the reference attends a repeated list entry repeatedly)
-  __shared__ int16_t ulist[2 * kMaxBlocksAttn];
+  // more than k times (the reference attends a repeated list entry repeatedly); then
+  // the tile's own block, one past two full lists with no entry in common
+  __shared__ int16_t ulist[2 * kMaxBlocksAttn + 1];
   __shared__ uint8_t uflag[2 * kMaxBlocksAttn];      // bit i: occurrence is item i's
   __shared__ uint32_t mult[2][kMaxBlocksAttn / 2];   // per-item times listed, 16 bits per block
   __shared__ float tail_bias[2][kTailTile];
