@@ -80,6 +80,18 @@ def _layer_shapes_match(query, key, value) -> bool:
             and tuple(key.shape) == (batch, kv_heads, sequence, head_dim))
 
 
+def _decode_shapes_fit(query, key, value) -> bool:
+    """Whether spx_decode_attention runs these [batch, head, sequence, dim] shapes: one
+    query row, nothing empty (an empty query included: the kernel has no grid for it), no
+    more keys than it counts."""
+    batch, q_heads, rows, head_dim = query.shape
+    shape = key.shape
+    return (rows == 1 and head_dim in (128, 256) and shape == value.shape
+            and 0 not in query.shape and 0 not in shape and shape[2] <= 1 << 30
+            and shape[0] == batch and shape[3] == head_dim and q_heads % shape[1] == 0
+            and batch * q_heads <= 65535)
+
+
 def _decode_kernel_takes(query, key, value, scaling) -> bool:
     """Whether a non-prefill call is a decode step of spx_decode_attention: one query
     row per head of plain bf16 GPU tensors in a layout it reads in place, and nothing
@@ -105,11 +117,7 @@ def _decode_kernel_takes(query, key, value, scaling) -> bool:
         batch, heads, rows, dim = x.stride()
         if dim != 1 or (batch | heads | rows) & 7 or x.data_ptr() & 15:
             return False
-    batch, q_heads, rows, head_dim = query.shape
-    shape = key.shape
-    if rows != 1 or head_dim not in (128, 256) or shape != value.shape or 0 in shape \
-            or shape[0] != batch or shape[3] != head_dim or q_heads % shape[1] \
-            or batch * q_heads > 65535:
+    if not _decode_shapes_fit(query, key, value):
         return False
     if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad
                                     or value.requires_grad):

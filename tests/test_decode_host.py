@@ -67,3 +67,20 @@ def test_prefill_scratch_needs_matching_shapes():
         assert not match(q, bad, bad) and not match(q, kv, bad) and not match(q, bad, kv)
     assert not match((0, 8, 300, 128), (0, 4, 300, 128), (0, 4, 300, 128))
     assert not match(q[1:], kv, kv)
+
+
+def test_decode_shapes():
+    """Calls that the decode kernel cannot run stay with SDPA, empty ones among them."""
+    def fit(q, k, v=None):
+        return attention._decode_shapes_fit(*(torch.empty(*s, device="meta") for s in (q, k, v or k)))
+
+    q, kv = (2, 8, 1, 128), (2, 4, 300, 128)
+    assert fit(q, kv) and fit((2, 8, 1, 256), (2, 4, 1, 256)) and fit((4095, 16, 1, 128), (4095, 2, 3, 128))
+    for empty in ((2, 0, 1, 128), (0, 8, 1, 128), (2, 8, 0, 128), (2, 8, 1, 0)):
+        assert not fit(empty, kv)
+    for bad in ((2, 0, 300, 128), (2, 4, 0, 128), (1, 4, 300, 128), (2, 3, 300, 128),
+                (2, 4, 300, 256)):
+        assert not fit(q, bad) and not fit(q, kv, bad)
+    assert not fit((2, 8, 2, 128), kv) and not fit((2, 8, 1, 64), (2, 4, 300, 64))
+    assert not fit((4096, 16, 1, 128), (4096, 2, 3, 128))       # 65536 rows
+    assert not fit((1, 1, 1, 128), (1, 1, (1 << 30) + 1, 128))
