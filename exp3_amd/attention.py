@@ -92,6 +92,15 @@ def _decode_shapes_fit(query, key, value) -> bool:
             and batch * q_heads <= 65535)
 
 
+def _reads_in_place(x) -> bool:
+    """Whether spx_decode_attention reads this tensor's storage as it is: a plain bf16
+    tensor, no lazy negation, 16-byte rows."""
+    if type(x) is not torch.Tensor or x.dtype is not torch.bfloat16 or x.dim() != 4 or x.is_neg():
+        return False
+    batch, heads, rows, dim = x.stride()
+    return dim == 1 and not (batch | heads | rows) & 7 and not x.data_ptr() & 15
+
+
 def _decode_kernel_takes(query, key, value, scaling) -> bool:
     """Whether a non-prefill call is a decode step of spx_decode_attention: one query
     row per head of plain bf16 GPU tensors in a layout it reads in place, and nothing
@@ -111,11 +120,7 @@ def _decode_kernel_takes(query, key, value, scaling) -> bool:
         return False
     device = torch._C._cuda_getDevice() if query.is_cuda else -2
     for x in (query, key, value):
-        if type(x) is not torch.Tensor or x.get_device() != device \
-                or x.dtype is not torch.bfloat16 or x.dim() != 4:
-            return False
-        batch, heads, rows, dim = x.stride()
-        if dim != 1 or (batch | heads | rows) & 7 or x.data_ptr() & 15:
+        if not _reads_in_place(x) or x.get_device() != device:
             return False
     if not _decode_shapes_fit(query, key, value):
         return False

@@ -84,3 +84,12 @@ def test_decode_shapes():
     assert not fit((2, 8, 2, 128), kv) and not fit((2, 8, 1, 64), (2, 4, 300, 64))
     assert not fit((4096, 16, 1, 128), (4096, 2, 3, 128))       # 65536 rows
     assert not fit((1, 1, 1, 128), (1, 1, (1 << 30) + 1, 128))
+
+
+def test_tensors_read_in_place():
+    reads = attention._reads_in_place
+    x = torch.zeros(2, 4, 40, 128, dtype=torch.bfloat16)
+    assert reads(x) and reads(x.transpose(1, 2)) and reads(x[:, :, 8:]) and reads(x.expand(2, 4, 40, 128))
+    assert not reads(torch._neg_view(x))          # negated when read, not in storage
+    assert not reads(x.half()) and not reads(x[0]) and not reads(x.transpose(2, 3))
+    assert not reads(x[..., 1:]) and not reads(torch.nn.Parameter(x))
