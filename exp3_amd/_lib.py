@@ -130,11 +130,16 @@ def strides(tensor: torch.Tensor | None):
     return STRIDES[len(values)](*values)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream(device: torch.device) -> int:
-    """The device's current stream (the raw handle: a torch Stream object costs 2 us
-    of the 12 to 60 us that a short call spends on the host)."""
+    """The device's current stream (the raw handle where torch gives it: a torch Stream
+    object costs 2 us of the 12 to 60 us that a short call spends on the host)."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     index = torch.cuda.current_device() if device.index is None else device.index
-    return torch._C._cuda_getCurrentRawStream(index)
+    return _raw_stream(index)
 
 
 def work_queue(batch, sequence, q_heads, kv_heads, head_dim, device):

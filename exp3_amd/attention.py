@@ -31,12 +31,20 @@ from __future__ import annotations
 import torch
 from torch.autograd import forward_ad
 import torch.nn.functional as F
-from torch.overrides import _get_current_function_mode_stack
-from torch.utils._device import DeviceContext
 
 from . import _lib, kernels
 from .kernels import BlockDescriptors
 from .upstream import flashprefill_native_forward as upstream
+
+try:
+    # torch has no public way to ask for the transforms and modes around a call
+    from torch.overrides import _get_current_function_mode_stack as _function_modes
+    from torch.utils._device import DeviceContext
+    _dispatch_modes = torch._C._len_torch_dispatch_stack
+    _transform_level = torch._C._functorch.maybe_current_level
+    forward_ad._current_level
+except (ImportError, AttributeError):
+    _function_modes = None     # a torch without these: decode steps stay with SDPA
 
 try:  # transformers is optional: the backend also runs standalone
     from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
@@ -109,16 +117,15 @@ def _decode_kernel_takes(query, key, value, scaling) -> bool:
     SDPA runs one workgroup per head (28/4 heads: 1156 us behind 32K tokens, 150 behind
     4K); at 130 tokens both are bound by the host's launches, so the length does not
     decide."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._functorch.maybe_current_level() is not None
-            or torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0
+    if (_function_modes is None or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or _transform_level() is not None or _dispatch_modes() or forward_ad._current_level >= 0
             or any(type(mode) is not DeviceContext       # a default device: factories only
-                   for mode in _get_current_function_mode_stack())
+                   for mode in _function_modes())
             or torch.is_autocast_enabled("cuda") or not torch.backends.cuda.flash_sdp_enabled()):
         return False
     if not isinstance(scaling, (int, float)):
         return False
-    device = torch._C._cuda_getDevice() if query.is_cuda else -2
+    device = torch.cuda.current_device() if query.is_cuda else -2
     for x in (query, key, value):
         if not _reads_in_place(x) or x.get_device() != device:
             return False

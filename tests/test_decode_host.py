@@ -2,6 +2,9 @@
 the C entry points refuse what they cannot run before any launch."""
 
 import ctypes
+from pathlib import Path
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -93,3 +96,35 @@ def test_tensors_read_in_place():
     assert not reads(torch._neg_view(x))          # negated when read, not in storage
     assert not reads(x.half()) and not reads(x[0]) and not reads(x.transpose(2, 3))
     assert not reads(x[..., 1:]) and not reads(torch.nn.Parameter(x))
+
+
+@pytest.mark.parametrize("missing", ("torch.overrides._get_current_function_mode_stack",
+                                     "torch.utils._device.DeviceContext",
+                                     "torch._C._len_torch_dispatch_stack",
+                                     "torch._C._functorch.maybe_current_level",
+                                     "torch.autograd.forward_ad._current_level"))
+def test_torch_without_private_names(missing):
+    """The backend imports and leaves its decode steps to SDPA."""
+    program = f"""
+import torch, torch.overrides, torch.utils._device, torch.autograd.forward_ad
+q, k = torch.randn(1, 4, 1, 128), torch.randn(1, 2, 40, 128)
+want = torch.nn.functional.scaled_dot_product_attention(q, k, k, scale=0.1, enable_gqa=True)
+del {missing}
+from exp3_amd import attention
+backend = attention.AttentionBackend(register=False)
+assert not attention._decode_kernel_takes(q, k, k, 0.1)
+out, _ = backend.forward(None, q, k, k, None, 0.1)
+assert torch.equal(out, want.transpose(1, 2))
+"""
+    done = subprocess.run([sys.executable, "-c", program], cwd=Path(__file__).resolve().parent.parent,
+                          capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr
+
+
+def test_stream_without_raw_handle(monkeypatch):
+    class Stream:
+        cuda_stream = 1234
+
+    monkeypatch.setattr(_lib, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: Stream)
+    assert _lib.stream(torch.device("cuda", 0)) == 1234
