@@ -782,8 +782,8 @@ __global__ __launch_bounds__(kSelectThreads) void mask_rows_kernel(MaskArgs a) {
                        a.counts, nullptr);
 }
 
-// The same with one workgroup per row, for more heads or key blocks than fit the LDS
-// words and lists of mask_rows_kernel.
+// The same with one workgroup per row: few rows, or more heads or key blocks than fit the
+// LDS words and lists of mask_rows_kernel.
 __global__ __launch_bounds__(kRouteThreads) void indices_from_mask_kernel(MaskArgs a) {
   const int h = blockIdx.x % a.heads;
   const int t = (blockIdx.x / a.heads) % a.query_blocks;
@@ -1036,7 +1036,15 @@ extern "C" int spx_indices_from_mask(const uint8_t* mask, int batch, int query_b
               "bad mask shape");
   MaskArgs a{const_cast<uint8_t*>(mask), batch, query_blocks, key_blocks, heads, indices, counts};
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (heads <= kSelectMaxHeads && key_blocks <= kMaxBlocks) {
+  // A workgroup per query tile pays with enough tiles to fill the CUs and enough heads
+  // that a line of 8-byte entries (16) is mostly its own. Kernel time, a workgroup per row
+  // -> per tile: 64 tiles x 300 keys, 8 heads 5.3 -> 4.8 us, 28 heads 9.2 -> 7.6, 256 x
+  // 256 at 28 heads 24 -> 7.5; below the line 64 x 300 at 4 heads 3.7 -> 4.4, 16 x 16 at
+  // 28 heads 3.2 -> 3.5, one tile x 1000 keys at 256 heads 8 -> 172, 1000 x 1000 at 2
+  // heads 11 -> 25.
+  const int64_t tiles = (int64_t)batch * query_blocks;
+  const bool by_tile = heads >= 6 && tiles >= 64 && tiles * heads >= 512;
+  if (by_tile && heads <= kSelectMaxHeads && key_blocks <= kMaxBlocks) {
     const int nch = (key_blocks + 63) / 64;
     const int grid = batch * query_blocks;
     constexpr int T = kSelectThreads;

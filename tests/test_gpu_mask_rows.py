@@ -1,7 +1,7 @@
-"""indices_from_mask by (batch, query tile) workgroups: chunk edges of the key blocks,
-head groups that exceed the LDS lists, and the sizes past its limits (256 heads, 1024 key
-blocks) that keep one workgroup per row; masks without any causal order, empty and full
-rows, bytes other than 0 and 1."""
+"""indices_from_mask by (batch, query tile) workgroups (64 tiles and 6 heads or more) and
+with one workgroup per row: chunk edges of the key blocks, head groups that exceed the LDS
+lists, and the sizes past the first form's limits (256 heads, 1024 key blocks); masks
+without any causal order, empty and full rows, bytes other than 0 and 1."""
 
 import pytest
 import torch
@@ -29,3 +29,44 @@ def test_lists_of_any_mask(gpu, batch, query, keys, heads):
         assert indices.dtype is torch.int64 and counts.dtype is torch.int32
         assert torch.equal(indices.cpu(), want)
         assert torch.equal(counts.cpu().long(), mask.sum(2))
+
+
+@pytest.mark.parametrize("batch,query,keys,heads", (
+    (1, 63, 63, 28), (1, 64, 1, 8), (2, 43, 64, 6), (2, 43, 65, 5), (1, 64, 65, 7), (3, 30, 129, 17),
+    (1, 64, 256, 32), (1, 70, 257, 9), (1, 65, 513, 28), (1, 64, 1024, 64), (1, 64, 1000, 256),
+    (1, 64, 130, 257), (1, 64, 1025, 8)))
+def test_lists_by_tile(gpu, batch, query, keys, heads):
+    gen = torch.Generator("cuda").manual_seed(keys * 5 + heads)
+    share = torch.rand(batch, query, 1, heads, generator=gen, device="cuda")
+    mask = torch.rand(batch, query, keys, heads, generator=gen, device="cuda") < share
+    mask[:, 0, :, 0] = False
+    mask[:, -1, :, -1] = True
+    ids = torch.arange(keys, device="cuda")[None, None, :, None]
+    want = torch.where(mask, ids, keys).sort(dim=2).values
+    value = torch.randint(1, 256, mask.shape, generator=gen, dtype=torch.uint8, device="cuda")
+    for given in (mask, value * mask):
+        indices, counts = kernels.indices_from_mask(given)
+        assert torch.equal(indices, want) and torch.equal(counts.long(), mask.sum(2))
+
+
+@pytest.mark.parametrize("shape", ((1, 2, 1024, 256), (1, 1, 1000, 64)))
+def test_few_tiles_use_the_chip(gpu, shape):
+    """One or two query tiles are spread over the CUs: 16 MB or less of lists within a few
+    times what it takes to fill them (one workgroup per tile: 4 to 40 times)."""
+    mask = torch.rand(shape, device="cuda") < 0.5
+    lists = torch.empty(shape, dtype=torch.int64, device="cuda")
+
+    def best(call):
+        times = []
+        for _ in range(10):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(20):
+                call()
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    # the call's own host work (two outputs, checks) is about two fills
+    assert best(lambda: kernels.indices_from_mask(mask)) <= 6 * best(lambda: lists.fill_(1))
