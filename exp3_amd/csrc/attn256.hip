@@ -566,7 +566,10 @@ __global__ __launch_bounds__(G * kA2Threads, 1) void attn256_kernel(Attn256Args 
 // routed, 1100 (144) 67 -> 60, 4500 (576) 196 -> 141, 6113 with rescue tokens (768) 289 ->
 // 225; 12/2 heads, 9000 (852) 357 -> 251. Beyond: 4 x 1300 (704, 11 blocks) 100 -> 116,
 // 4 x 2900 (1472) 253 -> 296, 12001 with every block (1504) 1040 -> 1089, routed 518 -> 417,
-// which the host cannot tell apart, 16000 dense (2000) 1771 -> 1845.
+// which the host cannot tell apart, 16000 dense (2000) 1771 -> 1845. A launch of tails
+// alone has no such chain (a step per 32 unlisted blocks) and stays with one group: block
+// means of 3000 tokens, 16/4 heads, 31 us against 44 with two (whole mean_tail calls), 300
+// tokens 17 against 22, 5000 55 against 62.
 constexpr int64_t kGroupItems = 384;
 constexpr int64_t kGroupItemsLong = 1024;
 constexpr int kGroupBlocksLong = 32;
@@ -618,8 +621,8 @@ int launch_attention_256(const Attn256Options& opt, const void* q, const int64_t
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t items = (int64_t)blocks * batch * q_heads;
-  const bool groups =
-      items <= kGroupItems || (items <= kGroupItemsLong && blocks >= kGroupBlocksLong);
+  const bool groups = opt.exact && (items <= kGroupItems ||
+                                    (items <= kGroupItemsLong && blocks >= kGroupBlocksLong));
   const int T = (groups ? 2 : 1) * kA2Threads;
   if (opt.exact && !opt.tail) {
     if (groups) attn256_kernel<true, false, false, 2><<<grid, T, 0, st>>>(a);
@@ -628,8 +631,7 @@ int launch_attention_256(const Attn256Options& opt, const void* q, const int64_t
     if (groups) attn256_kernel<true, true, false, 2><<<grid, T, 0, st>>>(a);
     else attn256_kernel<true, true, false, 1><<<grid, T, 0, st>>>(a);
   } else {
-    if (groups) attn256_kernel<false, true, true, 2><<<grid, T, 0, st>>>(a);
-    else attn256_kernel<false, true, true, 1><<<grid, T, 0, st>>>(a);
+    attn256_kernel<false, true, true, 1><<<grid, T, 0, st>>>(a);
   }
   return launch_status("attention_d256");
 }

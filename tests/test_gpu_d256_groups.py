@@ -7,7 +7,7 @@ with entries outside the sequence, and every method's tail."""
 import pytest
 import torch
 
-from exp3_amd import attention, synthetic
+from exp3_amd import attention, kernels, synthetic
 from exp3_amd.upstream import flashprefill_native_forward as upstream
 
 pytestmark = pytest.mark.gpu
@@ -71,3 +71,23 @@ def test_layers(gpu, method, length):
     out, _ = backend.forward(Layer(), *args, None, DIM ** -0.5)
     many, _ = backend.forward(Layer(), *(_batch(x) for x in args), None, DIM ** -0.5)
     _assert_close(out[0], many[-1], v)
+
+
+@pytest.mark.parametrize("length,seen", ((700, 1), (5000, 0), (5000, 3)))
+def test_tails_alone(gpu, length, seen):
+    """A launch of tails without exact blocks keeps one group (two were slower): the same
+    bits alone and in a batch, with tails of one and of several steps."""
+    q, k, v = _inputs(length, 8)
+    blocks = (length + 127) // 128
+    ids = torch.arange(blocks, device="cuda")
+    near = (ids[None, :] <= ids[:, None]) & (ids[:, None] - ids[None, :] < seen)
+    selected = near[None, :, :, None].expand(1, blocks, blocks, HEADS).contiguous()
+
+    def tails(q, k, v, selected):
+        return (kernels.mean_tail(q, kernels.block_descriptors(k, v), selected, DIM ** -0.5)
+                + kernels.rescue_tail(q, k, v, selected, DIM ** -0.5, remainder=True))
+
+    copies = 3 if length > 4096 else LONG     # past 1024 (tile, head) items
+    many = tails(*(x.expand(copies, *x.shape[1:]).contiguous() for x in (q, k, v, selected)))
+    for one, batch in zip(tails(q, k, v, selected), many):
+        assert torch.equal(one[0], batch[0]) and torch.equal(one[0], batch[-1])
