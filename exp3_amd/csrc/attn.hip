@@ -992,8 +992,10 @@ struct AttnRequest {
 // Persistent grid: the last third of the tile pairs (the lightest: their lists are
 // the shortest) form the shared tail.
 constexpr int kStaticThirds = 2;
-// Steals with more streams than XCDs: from this many static items per workgroup on.
-constexpr int kStealItems = 4;
+// Steals: from this many static items per workgroup on, in quarters, with at least an
+// XCD for each stream, and with more streams than XCDs.
+constexpr int kStealQuarters = 7;
+constexpr int kStealQuartersMixed = 16;
 
 // Workgroups per XCD of the persistent grid: one per CU (the kernel's LDS and
 // registers admit one workgroup per CU).
@@ -1132,14 +1134,19 @@ int launch_attention(const AttnRequest& req, const void* q, const int64_t* q_str
     while (tp0 > 0 && a.xcds_per_stream > 1 && (tp0 * a.group) % a.xcds_per_stream) --tp0;
     a.queue = req.work_queue;
     a.static_tp = tp0;
-    // Steals pay as soon as an XCD serves one stream (28/4 heads, routed lists: 6000
-    // tokens 211 -> 204 us, 16000 799 -> 689 us; every block listed: no change). With
-    // more streams than XCDs each XCD already mixes several, and the look at the counters
-    // that ends each workgroup costs more than it finds until a share is several items
-    // per workgroup (32/8 heads: 4 x 2113 tokens, 3 items, 225 -> 227 us; 4 x 4500
-    // tokens, 6 items, 546 -> 534 us; 2 x 9000, 6 items, 831 -> 730 us).
-    a.steal = a.xcds_per_stream > 1 ||
-              tp0 * streams / 8 * a.group > kStealItems * persistent_per_xcd();
+    // A steal looks at the counters first, all in one cache line that every workgroup
+    // draws from. That pays where shares are uneven and long: an XCD or more per stream,
+    // 28/4 heads, routed lists, 6000 tokens (1.75 items) 211 -> 204 us, 16000 799 -> 689.
+    // Shorter launches have little to move (routed layers of 3100 to 5000 tokens: the same
+    // to 2 % with and without) and lose where lists are alike (random, 15 % of the blocks,
+    // kernel without -> with: 3100 tokens 41 -> 48 us, 5000 62 -> 72, 12/2 heads 7500 63 ->
+    // 71; at 6000 still 76 -> 81, against 5 % of a routed layer there). With more streams than XCDs each XCD already mixes several (32/8 heads: 4
+    // x 2113 tokens, 3 items, 225 -> 227 us; 4 x 4500 tokens, 6 items, 546 -> 534 us; 2 x
+    // 9000, 6 items, 831 -> 730 us).
+    const int share = a.xcds_per_stream > 1 ? tp0 * a.group / a.xcds_per_stream
+                                            : tp0 * streams / 8 * a.group;
+    a.steal = a.xcds_per_stream > 1 ? 4 * share >= kStealQuarters * persistent_per_xcd()
+                                    : 4 * share > kStealQuartersMixed * persistent_per_xcd();
     a.share_items = tp0 * a.group / a.xcds_per_stream;
     a.dyn_items = (np - tp0) * a.group * (a.xcds_per_stream > 1 ? 1 : streams);
     grid = 8 * std::min(persistent_per_xcd(), per_xcd);
