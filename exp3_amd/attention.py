@@ -45,6 +45,7 @@ try:
     forward_ad._current_level
 except (ImportError, AttributeError):
     _function_modes = None     # a torch without these: decode steps stay with SDPA
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 try:  # transformers is optional: the backend also runs standalone
     from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
@@ -89,24 +90,27 @@ def _layer_shapes_match(query, key, value) -> bool:
 
 
 def _decode_shapes_fit(query, key, value) -> bool:
-    """Whether spx_decode_attention runs these [batch, head, sequence, dim] shapes: one
-    query row, nothing empty (an empty query included: the kernel has no grid for it), no
-    more keys than it counts."""
-    batch, q_heads, rows, head_dim = query.shape
-    shape = key.shape
-    return (rows == 1 and head_dim in (128, 256) and shape == value.shape
-            and 0 not in query.shape and 0 not in shape and shape[2] <= 1 << 30
-            and shape[0] == batch and shape[3] == head_dim and q_heads % shape[1] == 0
-            and batch * q_heads <= 65535)
+    """Whether spx_decode_attention runs tensors of these [batch, head, sequence, dim]
+    shapes: one query row, nothing empty (an empty query included: the kernel has no grid
+    for it), no more keys than it counts."""
+    batch, q_heads, rows, head_dim = query
+    k_batch, kv_heads, keys, k_dim = key
+    return (rows == 1 and (head_dim == 128 or head_dim == 256) and key == value
+            and k_batch == batch > 0 and k_dim == head_dim and kv_heads > 0 and q_heads > 0
+            and 0 < keys <= 1 << 30 and q_heads % kv_heads == 0 and batch * q_heads <= 65535)
 
 
-def _reads_in_place(x) -> bool:
-    """Whether spx_decode_attention reads this tensor's storage as it is: a plain bf16
-    tensor, no lazy negation, 16-byte rows."""
-    if type(x) is not torch.Tensor or x.dtype is not torch.bfloat16 or x.dim() != 4 or x.is_neg():
-        return False
-    batch, heads, rows, dim = x.stride()
-    return dim == 1 and not (batch | heads | rows) & 7 and not x.data_ptr() & 15
+def _reads_in_place(tensors, device) -> bool:
+    """Whether spx_decode_attention reads these tensors' storage as it is: plain bf16
+    tensors of this device index, no lazy negation, 16-byte rows."""
+    for x in tensors:
+        if type(x) is not torch.Tensor or x.get_device() != device \
+                or x.dtype is not torch.bfloat16 or x.dim() != 4 or x.is_neg():
+            return False
+        batch, heads, rows, dim = x.stride()
+        if dim != 1 or (batch | heads | rows) & 7 or x.data_ptr() & 15:
+            return False
+    return True
 
 
 def _decode_kernel_takes(query, key, value, scaling) -> bool:
@@ -119,22 +123,16 @@ def _decode_kernel_takes(query, key, value, scaling) -> bool:
     decide."""
     if (_function_modes is None or torch.compiler.is_compiling() or torch.jit.is_tracing()
             or _transform_level() is not None or _dispatch_modes() or forward_ad._current_level >= 0
-            or any(type(mode) is not DeviceContext       # a default device: factories only
-                   for mode in _function_modes())
             or torch.is_autocast_enabled("cuda") or not torch.backends.cuda.flash_sdp_enabled()):
         return False
-    if not isinstance(scaling, (int, float)):
-        return False
-    device = torch.cuda.current_device() if query.is_cuda else -2
-    for x in (query, key, value):
-        if not _reads_in_place(x) or x.get_device() != device:
+    for mode in _function_modes():
+        if type(mode) is not DeviceContext:      # a default device: factories only
             return False
-    if not _decode_shapes_fit(query, key, value):
-        return False
-    if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad
-                                    or value.requires_grad):
-        return False
-    return True
+    return (isinstance(scaling, (int, float)) and query.is_cuda
+            and _reads_in_place((query, key, value), _current_device())
+            and _decode_shapes_fit(query.shape, key.shape, value.shape)
+            and not (torch.is_grad_enabled() and (query.requires_grad or key.requires_grad
+                                                  or value.requires_grad)))
 
 
 class AttentionBackend:

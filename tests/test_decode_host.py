@@ -75,7 +75,7 @@ def test_prefill_scratch_needs_matching_shapes():
 def test_decode_shapes():
     """Calls that the decode kernel cannot run stay with SDPA, empty ones among them."""
     def fit(q, k, v=None):
-        return attention._decode_shapes_fit(*(torch.empty(*s, device="meta") for s in (q, k, v or k)))
+        return attention._decode_shapes_fit(*(torch.Size(s) for s in (q, k, v or k)))
 
     q, kv = (2, 8, 1, 128), (2, 4, 300, 128)
     assert fit(q, kv) and fit((2, 8, 1, 256), (2, 4, 1, 256)) and fit((4095, 16, 1, 128), (4095, 2, 3, 128))
@@ -90,10 +90,13 @@ def test_decode_shapes():
 
 
 def test_tensors_read_in_place():
-    reads = attention._reads_in_place
+    def reads(x):
+        return attention._reads_in_place((x,), -1)       # the index of a CPU tensor
+
     x = torch.zeros(2, 4, 40, 128, dtype=torch.bfloat16)
     assert reads(x) and reads(x.transpose(1, 2)) and reads(x[:, :, 8:]) and reads(x.expand(2, 4, 40, 128))
     assert not reads(torch._neg_view(x))          # negated when read, not in storage
+    assert not attention._reads_in_place((x,), 0)
     assert not reads(x.half()) and not reads(x[0]) and not reads(x.transpose(2, 3))
     assert not reads(x[..., 1:]) and not reads(torch.nn.Parameter(x))
 
