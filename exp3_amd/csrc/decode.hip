@@ -295,14 +295,18 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_merge_kernel(DecodeArgs
 // ranges to merge, so that short caches still use many CUs. Up to two steps run as one
 // workgroup per stream without the merge launch: 512 keys (28/4 heads) 13.0 us against
 // 10.7 us plus the second launch's 3.5 us of host time (eager 13.1 against 16.3 us), the
-// host being the bound there.
+// host being the bound there. So do three steps where only two ranges per stream fit, and
+// four from three workgroups for each two residents on: cut in two, the ranges are uneven
+// and in two rounds (8/8 heads, 64 sequences: 520 keys 43 us in two ranges, 31 in one, 800
+// keys 47 and 40; SDPA 30 and 40. 48 sequences: 600 keys 34 and 31; 1024 keys 47 and 49).
 template <int D>
 void decode_ranges(int batch, int seq, int q_heads, int kv_heads, int& splits, int& steps) {
   const int64_t units = (seq + DecodeShape<D>::kStepKeys - 1) / DecodeShape<D>::kStepKeys;
   const int tiles = (q_heads / kv_heads + kDecodeHeads - 1) / kDecodeHeads;
   const int64_t streams = (int64_t)batch * kv_heads * tiles;
   const int64_t most = std::min<int64_t>(kDecodeMaxSplits, std::max<int64_t>(1, 1024 / streams));
-  steps = (int)std::max<int64_t>((units + most - 1) / most, units <= 2 ? units : 1);
+  const int whole = most == 2 ? (streams > 384 ? 4 : 3) : 2;   // steps run as one range
+  steps = (int)std::max<int64_t>((units + most - 1) / most, units <= whole ? units : 1);
   splits = (int)((units + steps - 1) / steps);
 }
 

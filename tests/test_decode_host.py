@@ -131,3 +131,13 @@ def test_stream_without_raw_handle(monkeypatch):
     monkeypatch.setattr(_lib, "_raw_stream", None)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device: Stream)
     assert _lib.stream(torch.device("cuda", 0)) == 1234
+
+
+def test_few_steps_of_many_streams_are_one_range():
+    """Three or four steps of a stream are not cut in two where the launch has a stream for
+    most workgroups (no workspace: one range)."""
+    size = _lib.load().spx_decode_workspace_bytes
+    assert size(64, 600, 8, 8, 128) == size(43, 700, 8, 8, 128) == size(49, 1000, 8, 8, 128) == 0
+    assert size(32, 300, 16, 16, 256) == size(128, 1024, 28, 4, 128) == 0
+    for streams, keys, ranges in ((42, 700, 3), (48, 1000, 2), (64, 1100, 2), (49, 1100, 2)):
+        assert size(streams, keys, 8, 8, 128) == ranges * streams * 8 * 130 * 4

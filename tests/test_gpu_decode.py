@@ -139,3 +139,11 @@ def test_what_stays_with_sdpa(gpu):
     out, _ = backend.forward(_Layer(), leaf.to(torch.bfloat16), k, v, None, 0.1)
     out.sum().backward()
     assert leaf.grad is not None and torch.isfinite(leaf.grad).all()
+
+
+# one range of three and of four steps per stream, whole and with a few keys in the last
+@pytest.mark.parametrize("batch,layout,length", ((64, (8, 8, 128), 514), (49, (8, 8, 128), 1024),
+                                                 (33, (32, 16, 256), 300), (26, (16, 16, 256), 511)))
+def test_one_range_of_several_steps(gpu, batch, layout, length):
+    q, k, v = _inputs(batch, *layout, length, seed=11, sharp=6.0)
+    _close(_step(q, k, v, layout[2] ** -0.5), _want(q, k, v, layout[2] ** -0.5))
