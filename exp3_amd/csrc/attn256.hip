@@ -557,22 +557,32 @@ __global__ __launch_bounds__(G * kA2Threads, 1) void attn256_kernel(Attn256Args 
         l > 0.0f ? (log2f(l) - neg_m) * kLn2 : -INFINITY;
 }
 
-// Launches of up to kGroupItems items, or kGroupItemsLong of at least kGroupBlocksLong
-// blocks, use two groups per tile. There the chain of the longest list decides; with
-// more items the work does, and two groups, which meet at a barrier every sub-block and
-// leave a CU one workgroup (nothing beside its lists, Q and output), lose. Layers, one ->
-// two groups, 16/4 heads: every block listed, 2900 tokens (368 items) 140 -> 106 us, 4100
-// (528) 201 -> 172, 5000 (640) 251 -> 240, 8192 (1024) 547 -> 527; 4 x 700 (384) 67 -> 61;
-// routed, 1100 (144) 67 -> 60, 4500 (576) 196 -> 141, 6113 with rescue tokens (768) 289 ->
-// 225; 12/2 heads, 9000 (852) 357 -> 251. Beyond: 4 x 1300 (704, 11 blocks) 100 -> 116,
-// 4 x 2900 (1472) 253 -> 296, 12001 with every block (1504) 1040 -> 1089, routed 518 -> 417,
-// which the host cannot tell apart, 16000 dense (2000) 1771 -> 1845. A launch of tails
-// alone has no such chain (a step per 32 unlisted blocks) and stays with one group: block
-// means of 3000 tokens, 16/4 heads, 31 us against 44 with two (whole mean_tail calls), 300
-// tokens 17 against 22, 5000 55 against 62.
-constexpr int64_t kGroupItems = 384;
-constexpr int64_t kGroupItemsLong = 1024;
-constexpr int kGroupBlocksLong = 32;
+// Whether a launch uses two groups per tile. They halve the chain of a long list and cost
+// an exchange per tile and a barrier every sub-block, and a CU holds one workgroup instead
+// of two. So they pay where the longest lists decide, not the work: few items, or few items
+// of a tile (the last tiles list every block) against its length. Layers, one -> two
+// groups, 16/4 heads, lists of the default protections (topics) and of every block:
+//   blocks 3, 48 items 39 -> 38 us; 6, 288 items 62 -> 57; 12, 384 items 95 -> 84; 24, 384
+//   items 143 -> 112 and 145 -> 121; 36, 576 items 204 -> 155 and 227 -> 222; 64, 1024
+//   items 345 -> 286 and 544 -> 552
+// and beyond: 1 and 2 blocks 28 -> 29.5 and 34 -> 34.5; 6 blocks, 384 items 67 -> 67.5; 32
+// blocks at 32 items a tile 219 -> 232 and 306 -> 322; 12 blocks, 576 items 104 -> 114.
+// Up to 1024 items every block listed may lose up to 7 % (48 blocks, 768 items 328 -> 345)
+// where routed lists gain 20: the host cannot tell them apart, nor lists shorter than the
+// default protections give, which lose most (its own block alone: 300 items 17 -> 25 us).
+// A launch of tails alone has no such chain (a step per 32 unlisted blocks) and stays with
+// one group: block means of 3000 tokens, 16/4 heads, 31 us against 44 with two (whole
+// mean_tail calls), 300 tokens 17 against 22, 5000 55 against 62.
+constexpr int64_t kGroupItems = 384, kGroupItemsShort = 320, kGroupItemsLong = 1024;
+constexpr int kGroupBlocks = 12, kGroupBlocksShort = 3, kGroupBlocksLong = 32;
+constexpr int64_t kGroupTileItems = 24;   // of long launches
+
+bool two_groups(int blocks, int64_t tile_items) {
+  const int64_t items = blocks * tile_items;
+  return (blocks >= kGroupBlocksShort && items <= kGroupItemsShort) ||
+         (blocks >= kGroupBlocks && items <= kGroupItems) ||
+         (blocks >= kGroupBlocksLong && items <= kGroupItemsLong && tile_items <= kGroupTileItems);
+}
 
 int launch_attention_256(const Attn256Options& opt, const void* q, const int64_t* q_strides,
                          const void* key_tiles, const void* value_tiles, const int64_t* indices,
@@ -620,9 +630,7 @@ int launch_attention_256(const Attn256Options& opt, const void* q, const int64_t
     grid = (unsigned)(a.static_ranks * batch * q_heads) + (unsigned)((a.dyn_items * 5 + 3) / 4);
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t items = (int64_t)blocks * batch * q_heads;
-  const bool groups = opt.exact && (items <= kGroupItems ||
-                                    (items <= kGroupItemsLong && blocks >= kGroupBlocksLong));
+  const bool groups = opt.exact && two_groups(blocks, (int64_t)batch * q_heads);
   const int T = (groups ? 2 : 1) * kA2Threads;
   if (opt.exact && !opt.tail) {
     if (groups) attn256_kernel<true, false, false, 2><<<grid, T, 0, st>>>(a);

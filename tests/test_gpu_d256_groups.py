@@ -1,7 +1,7 @@
 """Head dim 256: short launches split each tile's keys over two groups of waves
 (csrc/attn256.hip), long ones do not. The same sequence alone and within a batch that
 makes the launch long: same lists, outputs and LSEs within the rounding of the
-probabilities, for one to four blocks, ragged ends, empty, unsorted and repeated lists
+probabilities, for one to four blocks (two groups from three on), ragged ends, empty, unsorted and repeated lists
 with entries outside the sequence, and every method's tail."""
 
 import pytest
@@ -91,3 +91,22 @@ def test_tails_alone(gpu, length, seen):
     many = tails(*(x.expand(copies, *x.shape[1:]).contiguous() for x in (q, k, v, selected)))
     for one, batch in zip(tails(q, k, v, selected), many):
         assert torch.equal(one[0], batch[0]) and torch.equal(one[0], batch[-1])
+
+
+@pytest.mark.parametrize("batch,length", ((1, 100), (1, 256), (4, 731), (2, 4059)))
+def test_where_one_group_stays(gpu, batch, length):
+    """One or two blocks, few blocks of many heads and sequences of a batch: the bits of
+    the one-group kernel."""
+    q, k, v = _inputs(length, 9)
+    blocks = (length + 127) // 128
+    idx = torch.arange(blocks, device="cuda")[None, None, :, None].expand(1, blocks, blocks, HEADS)
+    cnt = torch.arange(1, blocks + 1, device="cuda", dtype=torch.int32)[None, :, None]
+    cnt = cnt.expand(1, blocks, HEADS)
+
+    def outputs(count):
+        args = (x.expand(count, *x.shape[1:]).contiguous() for x in (q, k, v, idx, cnt))
+        return upstream.exact_attention(*args, DIM ** -0.5)
+
+    many = outputs(5 if length > 4000 else LONG)
+    for one, all_ in zip(outputs(batch), many):
+        assert torch.equal(one[0], all_[0]) and torch.equal(one[-1], all_[-1])
