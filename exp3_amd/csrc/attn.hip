@@ -1023,13 +1023,16 @@ int persistent_per_xcd() {
 // 117-161; 32/8 heads 2500 tokens (320) 92-95 -> 82-88, 3072 (384) 105-113 -> 96-115;
 // 12/2 heads 6500 tokens (312) 171-184 -> 150-170; by length, with items in plenty: 8 x
 // 400 tokens, 32/8 heads, 71 -> 62 us, 8 x 1089 165 -> 150, 8 x 1500 (12 blocks) 231-235
-// -> 217-227, 8 x 2048 (16 blocks) 333-361 -> 319-364.
-constexpr int kSoloBlocks = 12;
+// -> 217-227, 8 x 2048 (16 blocks) 333-361 -> 319-364. Without heads that share K and V the
+// second copy is not in the L2: 8/8 heads, every block listed, kernel, 80 x 1507 tokens
+// 540 -> 619, 30 x 995 (8 blocks) 101 -> 108, 32/32 heads, 30 x 867 (7) 353 -> 372, up to 6
+// blocks 0.7 to 1.02 of the pairs' time.
+constexpr int kSoloBlocks = 12, kSoloBlocksUnshared = 6;
 
-bool single_tiles(int batch, int seq, int q_heads) {
+bool single_tiles(int batch, int seq, int q_heads, int kv_heads) {
   const int blocks = num_blocks(seq);
   const int64_t pair_items = (int64_t)((blocks + 1) / 2) * batch * q_heads;
-  return blocks <= kSoloBlocks || pair_items * 3 <= persistent_per_xcd() * 8 * 4;
+  return blocks <= (q_heads > kv_heads ? kSoloBlocks : kSoloBlocksUnshared) || pair_items * 3 <= persistent_per_xcd() * 8 * 4;
 }
 
 int launch_attention(const AttnRequest& req, const void* q, const int64_t* q_strides,
@@ -1122,7 +1125,7 @@ int launch_attention(const AttnRequest& req, const void* q, const int64_t* q_str
       : (a.num_pairs + 7) / 8 * a.group;
   a.static_tp = np;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (!req.work_queue && req.exact && single_tiles(batch, seq, q_heads)) {
+  if (!req.work_queue && req.exact && single_tiles(batch, seq, q_heads, kv_heads)) {
     launch_attn_solo(a, req.tail, st);
     return launch_status("attention");
   }
@@ -1162,7 +1165,7 @@ int launch_attention(const AttnRequest& req, const void* q, const int64_t* q_str
 extern "C" int64_t spx_attention_queue_ints(int batch, int seq, int q_heads, int kv_heads,
                                             int head_dim) {
   if (batch <= 0 || seq <= 0 || kv_heads <= 0 || q_heads <= 0) return SPX_WORK_QUEUE_INTS;
-  return head_dim == kHeadDim && single_tiles(batch, seq, q_heads) ? 0 : SPX_WORK_QUEUE_INTS;
+  return head_dim == kHeadDim && single_tiles(batch, seq, q_heads, kv_heads) ? 0 : SPX_WORK_QUEUE_INTS;
 }
 
 extern "C" int spx_exact_attention(const void* q, const int64_t* q_strides,
