@@ -994,7 +994,7 @@ struct AttnRequest {
 constexpr int kStaticThirds = 2;
 // Steals: from this many static items per workgroup on, in quarters, with at least an
 // XCD for each stream, and with more streams than XCDs.
-constexpr int kStealQuarters = 7;
+constexpr int kStealQuarters = 6;
 constexpr int kStealQuartersMixed = 16;
 
 // Workgroups per XCD of the persistent grid: one per CU (the kernel's LDS and
@@ -1139,13 +1139,14 @@ int launch_attention(const AttnRequest& req, const void* q, const int64_t* q_str
     a.static_tp = tp0;
     // A steal looks at the counters first, all in one cache line that every workgroup
     // draws from. That pays where shares are uneven and long: an XCD or more per stream,
-    // 28/4 heads, routed lists, 6000 tokens (1.75 items) 211 -> 204 us, 16000 799 -> 689.
+    // 28/4 heads, routed lists, 6000 tokens (1.75 items) 211 -> 204 us, 16000 799 -> 689;
+    // 12/2 heads, 13730 tokens (1.7), heads of very different lists, 440 -> 404.
     // Shorter launches have little to move (routed layers of 3100 to 5000 tokens: the same
     // to 2 % with and without) and lose where lists are alike (random, 15 % of the blocks,
     // kernel without -> with: 3100 tokens 41 -> 48 us, 5000 62 -> 72, 12/2 heads 7500 63 ->
-    // 71; at 6000 still 76 -> 81, against 5 % of a routed layer there). With more streams than XCDs each XCD already mixes several (32/8 heads: 4
-    // x 2113 tokens, 3 items, 225 -> 227 us; 4 x 4500 tokens, 6 items, 546 -> 534 us; 2 x
-    // 9000, 6 items, 831 -> 730 us).
+    // 71; at 6000 still 76 -> 81). With more streams than XCDs each XCD already mixes
+    // several (32/8 heads: 4 x 2113 tokens, 3 items, 225 -> 227 us; 4 x 4500 tokens, 6
+    // items, 546 -> 534 us; 2 x 9000, 6 items, 831 -> 730 us).
     const int share = a.xcds_per_stream > 1 ? tp0 * a.group / a.xcds_per_stream
                                             : tp0 * streams / 8 * a.group;
     a.steal = a.xcds_per_stream > 1 ? 4 * share >= kStealQuarters * persistent_per_xcd()
