@@ -7,7 +7,7 @@ with entries outside the sequence, and every method's tail."""
 import pytest
 import torch
 
-from exp3_amd import attention, kernels, synthetic
+from exp3_amd import _lib, attention, kernels, synthetic
 from exp3_amd.upstream import flashprefill_native_forward as upstream
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +110,48 @@ def test_where_one_group_stays(gpu, batch, length):
     many = outputs(5 if length > 4000 else LONG)
     for one, all_ in zip(outputs(batch), many):
         assert torch.equal(one[0], all_[0]) and torch.equal(one[-1], all_[-1])
+
+
+@pytest.mark.parametrize("kind,q_heads,kv_heads,length", (("rescue2", 16, 4, 6113),
+                                                          ("rescue1", 12, 2, 10800),
+                                                          ("mean", 12, 2, 10800)))
+def test_several_tail_steps(gpu, kind, q_heads, kv_heads, length):
+    """Two groups take 32 tail entries each per step: sparse lists with up to 85 unlisted
+    blocks make two and three steps. Alone (two groups) against a batch of two (one)."""
+    q, k, v, _ = synthetic.make_inputs(length, seed=13, q_heads=q_heads, kv_heads=kv_heads,
+                                       head_dim=DIM, device="cuda")
+    q, k = (q.float() * 4).bfloat16(), (k.float() * 4).bfloat16()
+    blocks = (length + 127) // 128
+    ids = torch.arange(blocks, device="cuda")
+    gen = torch.Generator("cuda").manual_seed(2)
+    keep = torch.rand(1, blocks, blocks, q_heads, generator=gen, device="cuda") < 0.04
+    keep &= (ids[None, :] <= ids[:, None])[None, :, :, None]
+    keep[:, blocks // 2] = False            # a tile of its tail alone
+    assert (ids[-1] - keep[0, -1].sum(0)).max() > 32 * 2 // (2 if kind == "rescue2" else 1)
+    results = []
+    for copies in (1, 2):
+        q_, k_, v_, keep_ = (x.expand(copies, *x.shape[1:]).contiguous() for x in (q, k, v, keep))
+        d = kernels.block_descriptors(k_, v_)
+        tiles = upstream.attention_tiles(k_, v_)
+        choice = kernels.rescue_choice(q_, tiles[0])
+        idx, cnt = kernels.indices_from_mask(keep_)
+        out = torch.full(q_.shape, float("nan"), dtype=q.dtype, device="cuda")
+        lse = torch.full(q_.shape[:3], float("nan"), device="cuda")
+        head = (_lib.ptr(q_), _lib.strides(q_), _lib.ptr(tiles[0]), _lib.ptr(tiles[1]),
+                _lib.ptr(idx), _lib.strides(idx), _lib.ptr(cnt), _lib.strides(cnt))
+        end = (copies, length, q_heads, kv_heads, DIM, 128, DIM ** -0.5, _lib.ptr(out),
+               _lib.strides(out), _lib.ptr(lse), _lib.strides(lse), None, _lib.stream(q.device))
+        if kind == "mean":
+            _lib.call("spx_sparse_attention_mean", *head, _lib.ptr(d.mean_k), _lib.ptr(d.mean_v),
+                      _lib.ptr(d.counts), *end)
+        else:
+            _lib.call("spx_sparse_attention_rescue", *head, _lib.ptr(choice), _lib.ptr(v_),
+                      _lib.strides(v_), _lib.ptr(d.mean_k), _lib.ptr(d.mean_v),
+                      int(kind == "rescue2"), *end)
+        results.append((out[-1], lse[-1]))
+    (two, two_lse), (one, one_lse) = results
+    assert not torch.isnan(one).any() and not torch.isnan(two).any()
+    _assert_close(two, one, v)
+    empty = torch.isinf(one_lse)
+    assert torch.equal(torch.isinf(two_lse), empty)
+    assert torch.allclose(two_lse[~empty], one_lse[~empty], rtol=1e-5, atol=1e-4)

@@ -2,8 +2,8 @@
 spx_attention_queue_ints answers with 0) against the tile-pair kernel (the same call with a
 queue): the same bits on ascending lists, at the edges of its rule (12 blocks; pair items
 up to 4/3 of the CUs) and of its loops (one block, a lone first tile, partial last blocks,
-64-key halves, tails of more than one 64-entry tile), exact, with block means and with
-rescue tokens, LSE included; and unordered, repeated and future entries and empty rows
+64-key halves, tails of more than one 64-entry tile; lists and tails past one, two and
+more positions per thread), exact, with block means and with rescue tokens, LSE included; and unordered, repeated and future entries and empty rows
 within rounding of it (the two add blocks in different orders there)."""
 
 import pytest
@@ -91,3 +91,34 @@ def test_lists_in_any_order(gpu, kind):
     assert err.max() <= 2.0 ** -7 * v.float().abs().max()
     finite = torch.isfinite(pair[1])
     assert (solo[1] - pair[1])[finite].abs().max() <= 1e-4
+
+
+@pytest.mark.parametrize("kind", ("exact", "mean", "rescue2"))
+@pytest.mark.parametrize("length,q_heads,share", ((40000, 2, 0.3), (87000, 1, 0.6), (87000, 1, 0.02)))
+def test_long_lists(gpu, kind, length, q_heads, share):
+    """Few heads keep single tiles up to hundreds of blocks: more than 256 list positions
+    and tail blocks, a thread taking several of each."""
+    q, k, v, blocks, d, choice = _case(1, length, q_heads, 1, 9)
+    gen = torch.Generator("cuda").manual_seed(length)
+    keep = torch.rand(1, blocks, blocks, q_heads, generator=gen, device="cuda") < share
+    ids = torch.arange(blocks, device="cuda")
+    keep &= (ids[None, :] <= ids[:, None])[None, :, :, None]
+    keep[:, -1] = True                      # every block of the last tile
+    idx, cnt = kernels.indices_from_mask(keep)
+    solo, pair = _both(kind, q, k, v, idx, cnt, d, choice)
+    assert not torch.isnan(solo[0]).any()
+    assert torch.equal(solo[0], pair[0]) and torch.equal(solo[1], pair[1])
+    # a sampled tile against float64: its listed keys alone
+    if kind == "exact":
+        t = blocks - 7
+        blocks_of = idx[0, t, :cnt[0, t, 0], 0]
+        tokens = (blocks_of[:, None] * 128 + torch.arange(128, device="cuda")).flatten()
+        rows = slice(t * 128, t * 128 + 128)
+        logits = q[0, rows, 0].double() @ k[0, tokens, 0].double().T * 128 ** -0.5
+        hidden = tokens[None, :] > torch.arange(t * 128, t * 128 + 128, device="cuda")[:, None]
+        logits = logits.masked_fill(hidden, float("-inf"))
+        want = torch.softmax(logits, -1).nan_to_num() @ v[0, tokens, 0].double()
+        # P rounds to bf16 (half a step, 2^-9 of every share), the output by half a step of
+        # itself, fp32 sums below that
+        bound = 2 ** -8 * (v.double().abs().max() + want.abs())
+        assert ((solo[0][0, rows, 0].double() - want).abs() <= bound).all()
