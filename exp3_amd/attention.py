@@ -293,7 +293,8 @@ class AttentionBackend:
         common_head = (_lib.ptr(q), _lib.strides(q), _lib.ptr(tiles[0]), _lib.ptr(tiles[1]),
                        _lib.ptr(indices), _lib.strides(indices), _lib.ptr(counts),
                        _lib.strides(counts))
-        # zeroed counters of the kernel's persistent grid (work items taken in turn)
+        # zeroed counters of the kernel's persistent grid (work items taken in turn); None
+        # for launches that run faster with a workgroup per item
         queue = _lib.work_queue(batch, sequence, q_heads, k.shape[2], head_dim, device)
         common_tail = (batch, sequence, q_heads, k.shape[2], head_dim, self.block_size,
                        float(scale), _lib.ptr(output), _lib.strides(output), _lib.ptr(lse),

@@ -43,7 +43,7 @@
 //     which keeps the XCDs' shares of the work equal. Given a work queue, the grid
 //     is persistent: one workgroup per CU takes its XCD's items in that order from
 //     a counter, then the light last third of the tile pairs from a shared one, then
-//     what is left of the other XCDs' items.
+//     (in launches of enough items) what is left of the other XCDs' items.
 #include <type_traits>
 
 #include "attn_solo.h"
@@ -117,16 +117,15 @@ __device__ __forceinline__ void accumulate_pv(const uint16_t* vb, WaveState& ws,
   }
 }
 
-// One exact block: full tiles use every key sub-block with no masking; on the
-// diagonal wave w only reaches sub-blocks 0 .. w (keys above its queries are
-// masked, sub-blocks beyond w are skipped entirely).
-template <int NMB, bool DIAG>
-__device__ __forceinline__ void exact_block(const uint16_t* kb, const uint16_t* vb, WaveState& ws,
-                                            float scale, int q_pos) {
+// A tile's own block: the NMB key sub-blocks that reach this wave's queries (0 .. w for
+// wave w of the tile), keys above a query masked.
+template <int NMB>
+__device__ __forceinline__ void diagonal_block(const uint16_t* kb, const uint16_t* vb,
+                                               WaveState& ws, float scale, int q_pos) {
   f32x16 s[4];
   bf16x8 pb[8];
   scores<NMB, false>(kb, ws, 0, s);
-  softmax<NMB, DIAG, false>(s, ws, scale, q_pos, nullptr, 0, pb);
+  softmax<NMB, true, false>(s, ws, scale, q_pos, nullptr, 0, pb);
   accumulate_pv<2 * NMB>(vb, ws, pb);
 }
 
@@ -185,15 +184,6 @@ __device__ __forceinline__ void sub_values(const OperandTables& tb, int j, bf16x
     for (int db = 0; db < 4; ++db)
       r[h * 4 + db] = lds_at(tb.v[2 * j + h] + BUF * kTileBytes + db * kRowGroupBytes);
 }
-
-// The copy of the next block: source tiles and the other buffers.
-struct NextCopy {
-  const uint16_t* k;
-  const uint16_t* v;
-  uint16_t* kd;
-  uint16_t* vd;
-  bool any;
-};
 
 // One full block in buffer BUF. The previous full block's last P V product
 // (value operands rv, probabilities pend) runs first, beside this block's first
@@ -404,13 +394,14 @@ __device__ __forceinline__ int static_share(const AttnArgs& a, int xcd) {
 // once it drew from it in vain (drawn).
 //
 // Order: own XCD's static share; the shared light tail, or with 8 / bg XCDs per stream
-// that of its own stream (whose K / V tiles its L2 holds); then, from one look at all
-// counters, the static share of another XCD with the most items left; then the other
-// tails. (Shares before the tail cost balanced layers a look at the counters per stolen
-// item: four 2113-token sequences 225 -> 231 us.) Routed lists differ in length from head
-// to head and group to group by far more than XCD speeds do: without the steals a layer
-// ended with the XCDs of its densest kv group alone (heads selecting 10 to 100 % of the
-// blocks: layer of 131072 tokens 78.0 -> 42.7 ms, of 32640 tokens 2.49 -> 1.84 ms).
+// that of its own stream (whose K / V tiles its L2 holds); then, where the launch steals
+// (launch_attention), from one look at all counters, the static share of another XCD with
+// the most items left; then the other tails. (Shares before the tail cost balanced layers
+// a look at the counters per stolen item: four 2113-token sequences 225 -> 231 us.) Routed
+// lists differ in length from head to head and group to group by far more than XCD speeds
+// do: without the steals a layer ended with the XCDs of its densest kv group alone (heads
+// selecting 10 to 100 % of the blocks: layer of 131072 tokens 78.0 -> 42.7 ms, of 32640
+// tokens 2.49 -> 1.84 ms).
 //
 // A draw past the end of another XCD's share is given back, and what a workgroup never
 // drew from its own share and the tails is drawn once when it ends, so the final
@@ -717,8 +708,8 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) rv[i] = bf16x8{};
     pend[0] = pend[1] = bf16x8{};
-    // Full blocks: publish block u, then run it while its successor is copied (by
-    // full_block, spread over its steps; here at once if this item skips block u).
+    // Full blocks: publish block u, issue the copy of its successor, then run block u while
+    // that lands.
     auto run_full = [&](int uu, auto buf) {
       constexpr int B = decltype(buf)::value;
       // list entries first (written before the loop): their LDS reads overlap the wait
@@ -727,15 +718,9 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
       const int jn = __builtin_amdgcn_readfirstlane(ulist[more ? uu + 1 : uu]);
       wait_tiles();
       block_sync();  // block uu visible to all; every wave is done with block uu - 1
-      NextCopy nx;
-      nx.any = more;
-      nx.k = kbase + jn * tile_elems;
-      nx.v = vbase + jn * tile_elems;
-      nx.kd = kbuf[B ^ 1];
-      nx.vd = vbuf[B ^ 1];
-      if (nx.any) {  // block uu + 1 lands in the other buffers during block uu's math
-        dma_tile(nx.k, nx.kd, tid);
-        dma_tile(nx.v, nx.vd, tid);
+      if (more) {  // block uu + 1 lands in the other buffers during block uu's math
+        dma_tile(kbase + jn * tile_elems, kbuf[B ^ 1], tid);
+        dma_tile(vbase + jn * tile_elems, vbuf[B ^ 1], tid);
       }
       if ((f >> item) & 1) full_block<B>(tables, ws, scale, rv, pend);
     };
@@ -759,10 +744,10 @@ __device__ __forceinline__ void attn_item(const AttnArgs& a, int pair, int hg) {
       const int cur = item ? other : n_full & 1;
       for (int k = item ? n_diag1 : n_diag0; k > 0; --k) {
         switch (wi) {  // wave wi reaches key sub-blocks 0 .. wi of the diagonal block
-          case 0: exact_block<1, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-          case 1: exact_block<2, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-          case 2: exact_block<3, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
-          default: exact_block<4, true>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          case 0: diagonal_block<1>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          case 1: diagonal_block<2>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          case 2: diagonal_block<3>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
+          default: diagonal_block<4>(kbuf[cur], vbuf[cur], ws, scale, q_pos); break;
         }
       }
     }

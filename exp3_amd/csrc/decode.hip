@@ -18,11 +18,11 @@
 //     shuffles, no rounding of P; the fp32 rate is enough (0.5 GFLOP at 32K).
 //   * The four waves' (max, sum, O) merge in LDS; with more than one split a second
 //     kernel merges the splits' fp32 partials.
-// Measured (28/4 heads, one sequence; SDPA, which runs one workgroup per head, before):
-// 32641 keys 1156 -> 19 us for both kernels (15.9 + 4.0; 67 MB at the 5.0 TB/s of a
-// device copy take 13.4), 131072 keys 4580 -> 53 us (floor 53.7), 4096 keys 150 -> 11 us
-// in a graph; 8 x 16000 keys at 32/8 heads 630 -> 104 us (floor 105); D = 256, 16/4
-// heads, 32641 keys 1660 -> 32 us (floor 26.7).
+// Measured (28/4 heads, one sequence; SDPA, which runs one workgroup per head, before; in
+// brackets the bytes at the 6.2 TB/s of a pass over 1 GB that only reads; a device copy
+// moves 5.0): 32641 keys 1156 -> 19 us for both kernels, 15.9 + 4.0 (10.8), 131072 keys
+// 4580 -> 53 us (43), 4096 keys 150 -> 11 us in a graph (1.4); 8 x 16000 keys at 32/8 heads
+// 630 -> 104 us (85); D = 256, 16/4 heads, 32641 keys 1660 -> 32 us (21.6).
 #include <algorithm>
 
 #include "common.h"
