@@ -51,8 +51,8 @@ def test_lists_by_tile(gpu, batch, query, keys, heads):
 
 @pytest.mark.parametrize("shape", ((1, 2, 1024, 256), (1, 1, 1000, 64)))
 def test_few_tiles_use_the_chip(gpu, shape):
-    """One or two query tiles are spread over the CUs: 16 MB or less of lists within a few
-    times what it takes to fill them (one workgroup per tile: 4 to 40 times)."""
+    """One or two query tiles are spread over the CUs: 4 MB or less of lists in a few times
+    what it takes to fill them (2 and 3 measured; with a workgroup per tile 13 and 60)."""
     mask = torch.rand(shape, device="cuda") < 0.5
     lists = torch.empty(shape, dtype=torch.int64, device="cuda")
 
@@ -68,5 +68,4 @@ def test_few_tiles_use_the_chip(gpu, shape):
             times.append(begin.elapsed_time(end))
         return min(times)
 
-    # the call's own host work (two outputs, checks) is about two fills
-    assert best(lambda: kernels.indices_from_mask(mask)) <= 6 * best(lambda: lists.fill_(1))
+    assert best(lambda: kernels.indices_from_mask(mask)) <= 9 * best(lambda: lists.fill_(1))
